@@ -967,7 +967,9 @@ static int emit_new(const ms_format_desc &f, const uint64_t *vals, const uint64_
                     uint64_t chunk, uint64_t extra_values, temps &sc, ms_col **out, uint64_t **d_append)
 {
     ms_col *c;
-    MS_TRY(new_col(f, m_bound + extra_values, out_capacity(f, m_bound + extra_values, chunk), sc.s, &c));
+    const bool emit = f.kind != MS_UNCOMPR && !xfmt(f.kind);   // launch_emit sets the meta itself
+    MS_TRY(new_col(f, m_bound + extra_values, out_capacity(f, m_bound + extra_values, chunk), sc.s, &c, nullptr,
+                   !emit));
     *d_append = &c->meta->aux[0];
     int rc;
     if (f.kind == MS_UNCOMPR) {
@@ -978,7 +980,7 @@ static int emit_new(const ms_format_desc &f, const uint64_t *vals, const uint64_
         rc = chunk == 0 ? launch_xfmt_compress(c, vals, d_m, m_bound, 0, sc)
                         : ms_fail(MS_ERR_INVALID, "no write-iterator for format kind %u", f.kind);
     } else {
-        rc = launch_emit(c, vals, d_m, m_bound, chunk, nullptr, sc);
+        rc = launch_emit(c, vals, d_m, m_bound, chunk, sc);
     }
     if (rc) {
         ms_col_free(c);
@@ -1135,8 +1137,8 @@ extern "C" int ms_morph(ms_col **out, const ms_format_desc *dst, const ms_col *i
         *out = c;
         return MS_OK;
     }
-    MS_TRY(new_col(*dst, nb, out_capacity(*dst, nb, 0), S(stream), &c));
-    int rc = xfmt(dst->kind) ? launch_xfmt_compress(c, vals, d_n, nb, 0, sc) : launch_emit(c, vals, d_n, nb, 0, nullptr, sc);
+    MS_TRY(new_col(*dst, nb, out_capacity(*dst, nb, 0), S(stream), &c, nullptr, xfmt(dst->kind)));
+    int rc = xfmt(dst->kind) ? launch_xfmt_compress(c, vals, d_n, nb, 0, sc) : launch_emit(c, vals, d_n, nb, 0, sc);
     if (rc) { ms_col_free(c); return rc; }
     *out = c;
     return MS_OK;

@@ -718,10 +718,9 @@ int launch_delta_carries(const ms_col *in, temps &sc)
 
 static uint32_t units_grid(uint64_t count_bound) { return grid_for(count_bound / 512 + 1, WAVES * 8ull, 2048); }
 
-// Workgroups of `kernel` that the device holds at once (occupancy per CU
-// times CUs), queried once per kernel: grid-stride kernels that prefetch
-// their next piece of work run best as one resident wave of workgroups.
-static uint32_t resident_grid(const void *kernel)
+// Occupancy per CU times CUs: grid-stride kernels that prefetch their next
+// piece of work run best as one resident wave of workgroups.
+uint32_t resident_grid(const void *kernel, uint32_t wg)
 {
     static std::mutex mu;
     static std::map<std::pair<int, const void *>, uint32_t> cache;
@@ -734,7 +733,7 @@ static uint32_t resident_grid(const void *kernel)
     int cus = 0, blocks = 0;
     uint32_t g = 2048;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, WG, 0) == hipSuccess && cus > 0 && blocks > 0)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, (int)wg, 0) == hipSuccess && cus > 0 && blocks > 0)
         g = (uint32_t)(cus * blocks);
     cache[key] = g;
     return g;
@@ -743,7 +742,7 @@ static uint32_t resident_grid(const void *kernel)
 // Grid of a grid-stride kernel over `items` pieces of one wave each.
 static uint32_t stride_grid(const void *kernel, uint64_t items)
 {
-    const uint32_t r = resident_grid(kernel);
+    const uint32_t r = resident_grid(kernel, WG);
     return grid_for(items, WAVES, r < 8192 ? r : 8192);
 }
 

@@ -12,6 +12,7 @@
 // scan places the blocks, and a pack kernel assembles each block's
 // interleaved words in LDS and writes payload, headers and the block index.
 #include "ms_kernels.h"
+#include "ms_lookback.hpp"
 
 namespace ms {
 
@@ -640,7 +641,7 @@ __global__ __launch_bounds__(WG) void k_pack_static(emit_layout l, const uint64_
 // behind the output when *d_flag (select_compr.h:209-250).
 __global__ __launch_bounds__(WG) void k_emit_tail(emit_layout l, const uint64_t *v, const uint64_t *d_m,
                                                   const uint64_t *start, const uint32_t *bws, ms_dev_meta *meta,
-                                                  uint64_t *d_append, uint64_t *carries, uint8_t *out,
+                                                  uint64_t *carries, uint8_t *out,
                                                   const uint64_t *d_total, const uint64_t *d_flag)
 {
     const emit_plan pl = plan_of(l, *d_m);
@@ -664,7 +665,6 @@ __global__ __launch_bounds__(WG) void k_emit_tail(emit_layout l, const uint64_t 
         meta->size_used = app_done ? app + 8 * (total - pl.m) : rest ? R + 8 * rest : C;
         meta->aux[0] = app;
         meta->aux[1] = R;
-        if (d_append) *d_append = app;
     }
     if (appending && afits) {
         uint64_t *dst = (uint64_t *)(out + app);
@@ -713,21 +713,439 @@ static emit_layout out_layout(ms_col *out, uint64_t chunk)
     return l;
 }
 
-int launch_emit(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, uint64_t m_bound, uint64_t chunk,
-                uint64_t *d_append, temps &sc)
+// ------------------------------------------------------------------
+// Single-pass emission of 8-lane 512-value blocks (every DEFAULT_* cascade
+// and dynamic_vbp_f<512, P, 8>): a block's offset depends on the widths of
+// all blocks before it, so sizes and packing used to read the values twice
+// (for_f three times: its references first).  Here a wave keeps 4 blocks
+// (2048 values, one delta tile) in registers and a workgroup's 32 blocks
+// are one tile of a look-back over the tiles' byte totals.  A tile is packed
+// into LDS before its offset is known, and written out a tile later: its
+// look-back runs when the workgroup's next tile has published its total, so
+// a workgroup does not wait for every earlier tile's values to arrive.
+// Bound by HBM (values read once, the image written once).  Measured, kernel
+// time of all passes before and of this one: dynamic_vbp_f of 2^27 values
+// 630 -> 277 us (4.9 TB/s), delta_f 547 -> 246 us, for_f of 10^8 values
+// 703 -> 208 us; without the deferred look-back 319 / 290 / 251 us, with
+// tiles of 16 blocks (4 waves) 342 / 303 / 239 us.
+// ------------------------------------------------------------------
+typedef unsigned long long op_u64x2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t OP_WAVES = 8;                 // waves per workgroup
+constexpr uint32_t OP_WB = 4;                    // blocks per wave
+constexpr uint32_t OP_TILE = OP_WAVES * OP_WB;   // blocks per tile
+constexpr uint32_t OP_B = 512, OP_S = 8;
+constexpr uint32_t OP_SLOT = 256;                // LDS words per block: codes of up to 32 bits
+
+// Maximum over the wave (a DPP reduction into lane 63), uniform.
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x)
+{
+#define MS_DPP_MAX(ctl, rows)                                                                              \
+    {                                                                                                      \
+        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctl, rows, 0xf, false);        \
+        x = y > x ? y : x;                                                                                 \
+    }
+    MS_DPP_MAX(0x111, 0xf)   // row_shr:1, 2, 4, 8: each row's maximum in its last lane
+    MS_DPP_MAX(0x112, 0xf)
+    MS_DPP_MAX(0x114, 0xf)
+    MS_DPP_MAX(0x118, 0xf)
+    MS_DPP_MAX(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
+    MS_DPP_MAX(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
+#undef MS_DPP_MAX
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Orders a wave's LDS accesses among its lanes (LDS serves one wave in order).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Thread (g, j) holds codes 8 g .. 8 g + 7 of lane j (at most 32 bits each):
+// 8 bw bits that start at byte g bw of the lane's stream.  They are ORed
+// into the block's words (cleared here), two codes at a time and with one
+// LDS atomic per word touched.
+__device__ __forceinline__ void op_pack(uint32_t bw, const uint64_t (&c)[8], unsigned long long *lds, uint32_t t)
+{
+    const uint32_t byte0 = (t >> 3) * bw;
+    for (uint32_t i = t; i < 4 * bw; i += 64) ((op_u64x2 *)lds)[i] = op_u64x2{0, 0};
+    wave_lds_sync();
+    unsigned long long *p = lds + (byte0 >> 3) * 8 + (t & 7);
+    uint32_t sh = (byte0 & 7) * 8;
+    uint64_t acc = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint64_t x = (uint64_t)(uint32_t)c[2 * q] | ((uint64_t)(uint32_t)c[2 * q + 1] << bw);
+        acc |= x << sh;
+        const uint32_t n = sh + 2 * bw;
+        if (n >= 64) {
+            atomicOr(p, (unsigned long long)acc);
+            p += 8;
+            acc = n > 64 ? x >> (64 - sh) : 0ull;        // n > 64 only with sh > 0
+        }
+        sh = n & 63;
+    }
+    if (sh) atomicOr(p, (unsigned long long)acc);
+    wave_lds_sync();
+}
+
+// Words of the launch's look-back state: the ticket counter, a word per
+// tile, then (a column-level dynamic_vbp_f) a page start per page.
+static uint64_t op_tiles(uint64_t nb_bound) { return nb_bound / OP_TILE + 1; }
+
+// The n blocks of 512 values at src into x (thread (g, j): codes 8 g .. of
+// lane j); `before` = lane j's value in front of them (delta_f, g = 0).
+template <uint32_t KIND>
+__device__ __forceinline__ void op_load(const uint64_t *src, uint32_t n, bool first, uint32_t t,
+                                        uint64_t (&x)[OP_WB][8], uint64_t &before)
+{
+    const uint64_t *p = src + (t >> 3) * 64 + (t & 7);
+#pragma unroll
+    for (uint32_t k = 0; k < OP_WB; k++) {
+#pragma unroll
+        for (uint32_t q = 0; q < 8; q++) x[k][q] = k < n ? gload(p + k * OP_B + q * 8) : 0ull;
+    }
+    before = KIND == MS_DELTA && n && !first && t < 8 ? gload(src - 8 + t) : 0ull;
+}
+
+__device__ __forceinline__ void op_copy(uint32_t bw, const unsigned long long *lds, uint8_t *dst, uint32_t t)
+{
+    // written once, more than the caches hold (283 -> 276 us for 2^27 values)
+    for (uint32_t i = t; i < 4 * bw; i += 64)
+        __builtin_nontemporal_store(((const op_u64x2 *)lds)[i], (op_u64x2 *)dst + i);
+}
+
+// A block of a wave that holds codes of more than 32 bits, which the LDS
+// slots have no room for: its values are read again (they are warm in the
+// caches) once its offset is known, two at a time so that this rare path
+// does not set the kernel's register budget.
+template <uint32_t KIND>
+__device__ __forceinline__ void op_wide_block(const uint64_t *src, bool first, uint64_t ref, uint32_t bw,
+                                              unsigned long long *lds, uint8_t *dst, uint32_t t)
+{
+    const uint32_t g = t >> 3, words = 8 * bw;
+    for (uint32_t i = t; i < words; i += 64) lds[i] = 0;
+    wave_lds_sync();
+    const uint64_t *p = src + g * 64 + (t & 7);
+    uint32_t bit = g * 8 * bw;
+#pragma unroll 1
+    for (uint32_t q = 0; q < 8; q += 2) {
+        const bool start = KIND == MS_DELTA && first && g == 0 && q == 0;   // no value in front
+        uint64_t a = gload(p + q * 8), b = gload(p + q * 8 + 8), before = 0;
+        if (KIND == MS_DELTA && !start) before = gload(p + q * 8 - 8);
+        if (KIND == MS_DELTA) {
+            b -= a;
+            a -= before;
+        }
+        if (KIND == MS_FOR) {
+            a -= ref;
+            b -= ref;
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < 2; h++) {
+            const uint64_t c = h ? b : a;
+            unsigned long long *w = lds + (bit >> 6) * 8 + (t & 7);
+            const uint32_t sh = bit & 63;
+            atomicOr(w, (unsigned long long)(c << sh));
+            if (sh + bw > 64) atomicOr(w + 8, (unsigned long long)(c >> (64 - sh)));
+            bit += bw;
+        }
+    }
+    wave_lds_sync();
+    op_copy(bw, lds, dst, t);
+    wave_lds_sync();
+}
+
+// refs_out: for_f's references, delta_f's tile carries (a wave's 4 blocks
+// are one tile).  The last tile writes the column's meta and the raw rest.
+template <uint32_t KIND>
+__global__ __launch_bounds__(OP_WAVES * 64, 4) void k_emit_onepass(emit_layout l, const uint64_t *v, const uint64_t *d_m,
+                                                                 uint64_t *state, uint64_t tiles_bound,
+                                                                 ms_dev_meta *meta, uint8_t *out, uint64_t *index,
+                                                                 uint64_t *refs_out)
+{
+    __shared__ __align__(16) unsigned long long s_words[OP_WAVES][OP_WB * OP_SLOT];
+    __shared__ uint64_t s_ref[4][OP_TILE], s_tile, s_base, s_page;   // s_ref: of the last tiles, in turn
+    __shared__ uint32_t s_tot[OP_WAVES];
+    const emit_plan pl = plan_of(l, *d_m);
+    const uint32_t t = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t g = t >> 3;
+    uint64_t *tiles = state + 1, *pages = tiles + tiles_bound;
+    const uint64_t ntiles = pl.nb ? (pl.nb + OP_TILE - 1) / OP_TILE : 1;
+    const bool paged = KIND == MS_DYNAMIC_VBP && l.K == 0;   // pages of many tiles
+    const uint32_t bpo = (uint32_t)l.bpo;                     // 1, 2 or 4
+    const uint32_t P = (uint32_t)l.P, FP = (uint32_t)l.FP, fpb = FP * bpo;
+    const auto first_of = [&](uint64_t tile) -> uint64_t { return tile * OP_TILE + w * OP_WB; };
+    const auto blocks_of = [&](uint64_t b0) -> uint32_t {    // blocks of a wave that starts at b0
+        return b0 >= pl.nb ? 0u : pl.nb - b0 < OP_WB ? (uint32_t)(pl.nb - b0) : OP_WB;
+    };
+    if (threadIdx.x == 0) s_tile = lb_ticket(state);
+    __syncthreads();
+    uint64_t tile = readlane64(s_tile, 0);   // uniform: addresses and branches stay scalar
+    __syncthreads();
+    if (tile >= ntiles) return;
+    uint64_t x[OP_WB][8], before;
+    op_load<KIND>(v + first_of(tile) * OP_B, blocks_of(first_of(tile)), first_of(tile) == 0, t, x, before);
+    // the packed tile that waits for its offset: its blocks' widths and
+    // headers, the bytes of the waves before this one and of the tile
+    uint64_t ptile = ~0ull;
+    uint32_t pbw[OP_WB] = {0, 0, 0, 0}, phdr[OP_WB] = {0, 0, 0, 0}, pmine = 0, ptotal = 0;
+    for (uint32_t turn = 0;; turn = (turn + 1) & 3) {
+        const bool have = tile < ntiles;
+        uint32_t bw[OP_WB] = {0, 0, 0, 0}, hdr[OP_WB] = {0, 0, 0, 0};
+        if (have) {
+            // the workgroup's next tile
+            if (threadIdx.x == 0) s_tile = lb_ticket(state);
+            const uint64_t b0 = first_of(tile);
+            const uint32_t n = blocks_of(b0);
+            if (KIND == MS_DELTA) {
+                // the code before a thread's first one is lane t - 8's last
+                // (of the previous block for g = 0)
+                if (n && g == 0) refs_out[b0 / OP_WB * 8 + t] = before;
+#pragma unroll
+                for (uint32_t k = 0; k < OP_WB; k++) {
+                    const uint64_t last = __shfl(x[k][7], (int)((t + 56) & 63), MS_WAVE);
+                    const uint64_t prev = g ? last : before;
+                    before = last;
+#pragma unroll
+                    for (uint32_t q = 7; q > 0; q--) x[k][q] -= x[k][q - 1];
+                    x[k][0] -= prev;
+                }
+            }
+            if (KIND == MS_FOR) {
+                // signed minimum per lane, then unsigned over the lanes (for.h:121-161)
+                int64_t sm[OP_WB];
+#pragma unroll
+                for (uint32_t k = 0; k < OP_WB; k++) {
+                    sm[k] = (int64_t)x[k][0];
+#pragma unroll
+                    for (uint32_t q = 1; q < 8; q++) sm[k] = (int64_t)x[k][q] < sm[k] ? (int64_t)x[k][q] : sm[k];
+                }
+                if (bpo >= 2) {
+                    sm[0] = sm[1] < sm[0] ? sm[1] : sm[0];
+                    sm[2] = sm[3] < sm[2] ? sm[3] : sm[2];
+                }
+                if (bpo == 4) sm[0] = sm[2] < sm[0] ? sm[2] : sm[0];
+                uint64_t ref = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < OP_WB; k++) {
+                    if ((k & (bpo - 1)) == 0) {
+#pragma unroll
+                        for (uint32_t o = 8; o < 64; o <<= 1) {
+                            const int64_t y = (int64_t)__shfl_xor((uint64_t)sm[k], (int)o, MS_WAVE);
+                            sm[k] = y < sm[k] ? y : sm[k];
+                        }
+                        uint64_t r = (uint64_t)sm[k];
+#pragma unroll
+                        for (uint32_t o = 1; o < 8; o <<= 1) {
+                            const uint64_t y = __shfl_xor(r, (int)o, MS_WAVE);
+                            r = y < r ? y : r;
+                        }
+                        ref = readlane64(r == ~0ull ? r - 1 : r, 0);
+                        if (t == 0 && k < n) {
+                            s_ref[turn][(w * OP_WB + k) / bpo] = ref;
+                            refs_out[(b0 + k) / bpo] = ref;
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t q = 0; q < 8; q++) x[k][q] -= ref;
+                }
+            }
+            // header bytes in front of the wave's blocks: page meta at every
+            // call of the inner layout, for_f's reference page (of at least
+            // 8 references) at its page's first block
+            const bool page0 = KIND == MS_DYNAMIC_VBP ? (paged ? lmod(b0, P) == 0 : true)
+                             : KIND == MS_FOR         ? (l.K || (b0 & (fpb - 1)) == 0) : false;
+            uint32_t bytes = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < OP_WB; k++) {
+                if (k >= n) continue;
+                uint64_t o = 1;
+#pragma unroll
+                for (uint32_t q = 0; q < 8; q++) o |= x[k][q];
+                bw[k] = wave_max_u32(64 - __clzll(o));
+                if (KIND == MS_DYNAMIC_VBP) hdr[k] = k == 0 && page0 ? P : 0;
+                else hdr[k] = ((k & (bpo - 1)) == 0 ? P : 0) + (KIND == MS_FOR && k == 0 && page0 ? 8 * FP : 0);
+                bytes += hdr[k] + OP_B / 8 * bw[k];
+            }
+            if (t == 0) s_tot[w] = bytes;
+        }
+        __syncthreads();
+        uint64_t next = ~0ull;
+        uint32_t mine = 0, total = 0;
+        if (have) {
+            next = readlane64(s_tile, 0);
+#pragma unroll
+            for (uint32_t i = 0; i < OP_WAVES; i++) {
+                if (i == w) mine = total;
+                total += __builtin_amdgcn_readfirstlane(s_tot[i]);
+            }
+            if (w == 0) lb_publish(tiles, tile, total);
+        }
+        if (w == 0 && ptile != ~0ull) {
+            const uint64_t base = lb_exclusive(tiles, ptile, ptotal);
+            uint64_t page = 0;
+            if (paged) {
+                // the page's first tile publishes where the page starts; its
+                // others (whose tickets are later) wait for that
+                const uint64_t pg = ldiv(first_of(ptile), P);
+                if (first_of(ptile) == pg * P) {
+                    page = base;
+                    if (t == 0) lb_store(pages + pg, base + 1);
+                } else {
+                    while ((page = lb_load(pages + pg)) == 0) __builtin_amdgcn_s_sleep(1);
+                    page--;
+                }
+            }
+            if (t == 0) {
+                s_base = base;
+                s_page = page;
+            }
+        }
+        __syncthreads();
+        if (ptile != ~0ull) {
+            const uint64_t tbase = readlane64(s_base, 0), page = readlane64(s_page, 0);
+            const uint64_t b0 = first_of(ptile);
+            const uint32_t n = blocks_of(b0), pturn = (turn + 3) & 3;
+            const bool wide = pbw[0] > 32 || pbw[1] > 32 || pbw[2] > 32 || pbw[3] > 32;
+            const bool page0 = phdr[0] > P;
+            uint64_t at = tbase + pmine;
+#pragma unroll
+            for (uint32_t k = 0; k < OP_WB; k++) {
+                if (k >= n) break;
+                const uint64_t b = b0 + k, off = at + phdr[k];
+                at = off + OP_B / 8 * pbw[k];
+                if (at > l.cap) {                       // uniform per wave
+                    if (t == 0) emit_overflow(l);
+                    continue;
+                }
+                if (wide) op_wide_block<KIND>(v + b * OP_B, b == 0,
+                                              KIND == MS_FOR ? s_ref[pturn][(w * OP_WB + k) / bpo] : 0ull, pbw[k],
+                                              s_words[w], out + off, t);
+                else op_copy(pbw[k], s_words[w] + k * OP_SLOT, out + off, t);
+                if (t == 0) index[b] = (off << 8) | pbw[k];
+                if (paged) {
+                    if (t == 0) out[page + lmod(b, P)] = (uint8_t)pbw[k];
+                } else if (phdr[k]) {
+                    // a call's page meta: its blocks are this wave's
+                    const uint32_t nin = KIND == MS_DYNAMIC_VBP ? n : bpo;
+                    uint64_t m = ~0ull;
+#pragma unroll
+                    for (uint32_t i = OP_WB; i-- > 0;)
+                        if (i >= k && i - k < nin) m = (m << 8) | pbw[i];
+                    uint64_t *mp = (uint64_t *)(out + off - P);
+                    for (uint32_t i = t; i < P / 8; i += 64) mp[i] = i ? ~0ull : m;
+                    if (KIND == MS_FOR && k == 0 && page0) {
+                        // reference page (for.h:207-233): its blocks are this
+                        // wave's (a write-iterator's call) or this tile's
+                        const uint64_t left = pl.nfb - b / bpo;
+                        const uint32_t nfp = l.K ? n / bpo : left < FP ? (uint32_t)left : FP;
+                        uint64_t *rp = (uint64_t *)(out + off - phdr[k]);
+                        for (uint32_t i = t; i < FP; i += 64)
+                            rp[i] = i < nfp ? s_ref[pturn][w * OP_WB / bpo + i] : (i == nfp ? ~0ull : 0ull);
+                    }
+                }
+            }
+            if (ptile == ntiles - 1) {
+                const uint64_t C = tbase + ptotal, R = ms_align64(C + l.gap), rest = pl.m - pl.m_c;
+                const bool fits = R + 8 * rest <= l.cap;
+                if (threadIdx.x == 0) {
+                    if (!fits) emit_overflow(l);
+                    meta->count = pl.m;
+                    meta->size_compr = C;
+                    meta->size_used = rest ? R + 8 * rest : C;
+                    meta->aux[0] = rest ? R + 8 * rest : R;   // the write-iterator's append offset
+                    meta->aux[1] = R;
+                }
+                if (fits)
+                    for (uint64_t i = threadIdx.x; i < rest; i += OP_WAVES * 64)
+                        ((uint64_t *)(out + R))[i] = v[pl.m_c + i];
+                if (paged && pl.nb && C <= l.cap)             // blocks the last page lacks
+                    for (uint64_t i = lmod(pl.nb - 1, P) + 1 + threadIdx.x; i < P; i += OP_WAVES * 64)
+                        out[page + i] = (uint8_t)MS_VBP_BW_NOBLOCK;
+            }
+        }
+        if (!have) return;
+        wave_lds_sync();   // the packed words go where the written ones were
+        if (bw[0] <= 32 && bw[1] <= 32 && bw[2] <= 32 && bw[3] <= 32) {
+#pragma unroll
+            for (uint32_t k = 0; k < OP_WB; k++)
+                if (bw[k]) op_pack(bw[k], x[k], s_words[w] + k * OP_SLOT, t);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < OP_WB; k++) {
+            pbw[k] = bw[k];
+            phdr[k] = hdr[k];
+        }
+        pmine = mine;
+        ptotal = total;
+        ptile = tile;
+        tile = next;
+        if (tile < ntiles)
+            op_load<KIND>(v + first_of(tile) * OP_B, blocks_of(first_of(tile)), first_of(tile) == 0, t, x, before);
+    }
+}
+
+// Clears an output's meta and a launch's look-back state.
+__global__ __launch_bounds__(WG) void k_emit_init(uint64_t *meta, uint64_t *state, uint64_t words)
+{
+    if (blockIdx.x == 0 && threadIdx.x < 32) meta[threadIdx.x] = 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * WG + threadIdx.x; i < words; i += (uint64_t)gridDim.x * WG) state[i] = 0;
+}
+
+// Layouts the single-pass emission takes: blocks of one wave's shape whose
+// page meta lies within a wave (or, column-level dynamic_vbp_f, in pages of
+// whole tiles) and whose reference pages lie within a tile.
+static bool onepass_ok(const emit_layout &l)
+{
+    if (l.leaf != MS_DYNAMIC_VBP || l.S != OP_S || l.B != OP_B || l.P % 64 || l.P > (1u << 24) || l.FP > (1u << 24) || l.cmap || l.cout) return false;
+    if (l.K != 0 && l.K != OP_WB * OP_B) return false;
+    if (l.kind == MS_DYNAMIC_VBP) return true;
+    if (l.bpo != 1 && l.bpo != 2 && l.bpo != 4) return false;
+    if (l.kind == MS_DELTA) return l.dstep == OP_S;
+    return l.kind == MS_FOR && l.E == OP_S && l.FP % 8 == 0 && (l.K != 0 || OP_TILE % (l.FP * l.bpo) == 0);
+}
+
+static int launch_emit_onepass(ms_col *out, const emit_layout &l, const uint64_t *d_v, const uint64_t *d_m,
+                               uint64_t m_bound, temps &sc)
+{
+    hipStream_t s = sc.s;
+    const uint64_t nb_bound = m_bound / l.B + 1, tiles = op_tiles(nb_bound);
+    const uint64_t words = 1 + tiles + (l.kind == MS_DYNAMIC_VBP && l.K == 0 ? nb_bound / l.P + 1 : 0);
+    if (out->index_cap < nb_bound - 1 || (l.kind == MS_FOR && out->refs_cap < m_bound / l.L) ||
+        (l.kind == MS_DELTA && out->refs_cap < (m_bound / MS_DELTA_TILE + 1) * 8))
+        return ms_fail(MS_ERR_CAPACITY, "emit: index capacity");
+    uint64_t *state = (uint64_t *)sc.get(words * 8);
+    if (!state) return ms_fail(MS_ERR_NOMEM, "emit scratch");
+    hipLaunchKernelGGL(k_emit_init, dim3(grid_for(words, WG * 4ull, 256)), dim3(WG), 0, s, (uint64_t *)out->meta,
+                       state, words);
+    MS_HIP(hipGetLastError());
+    auto k = l.kind == MS_DYNAMIC_VBP ? k_emit_onepass<MS_DYNAMIC_VBP>
+           : l.kind == MS_DELTA       ? k_emit_onepass<MS_DELTA>
+                                      : k_emit_onepass<MS_FOR>;
+    const uint32_t resident = resident_grid((const void *)k, OP_WAVES * 64);
+    hipLaunchKernelGGL(k, dim3(grid_for(tiles, 1, resident)), dim3(OP_WAVES * 64), 0, s, l, d_v, d_m, state, tiles,
+                       out->meta, out->data, out->index, out->refs);
+    MS_HIP(hipGetLastError());
+    return MS_OK;
+}
+
+int launch_emit(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, uint64_t m_bound, uint64_t chunk, temps &sc)
 {
     hipStream_t s = sc.s;
     const ms_format_desc &f = out->f;
     const emit_layout l = out_layout(out, chunk);
     if (f.kind != MS_STATIC_VBP && l.B * 8 > 65536)
         return ms_fail(MS_ERR_INVALID, "emit: innermost blocks above 8192 values are not supported");
+    if (onepass_ok(l)) return launch_emit_onepass(out, l, d_v, d_m, m_bound, sc);
+    MS_TRY(launch_fill_u64((uint64_t *)out->meta, 32, 0, s));
     const uint64_t nb_bound = m_bound / l.B + 1;
     if (f.kind == MS_STATIC_VBP) {
         hipLaunchKernelGGL(k_pack_static, dim3(grid_for(m_bound * l.bw / 64 + 1, WG * 4ull)), dim3(WG), 0, s, l, d_v,
                            d_m, out->data);
         MS_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_emit_tail, dim3(grid_for(l.bs + l.K + 1, WG, 64)), dim3(WG), 0, s, l, d_v, d_m,
-                           (const uint64_t *)nullptr, (const uint32_t *)nullptr, out->meta, d_append,
+                           (const uint64_t *)nullptr, (const uint32_t *)nullptr, out->meta,
                            (uint64_t *)nullptr, out->data, (const uint64_t *)nullptr, (const uint64_t *)nullptr);
     } else {
         uint64_t *sz = (uint64_t *)sc.get(nb_bound * 8 + 64);
@@ -758,7 +1176,7 @@ int launch_emit(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, uint64_t 
             return ms_fail(MS_ERR_CAPACITY, "emit: delta carries capacity");
         const uint64_t tail = std::max<uint64_t>(l.bs + l.K + 1, m_bound / MS_DELTA_TILE * 8 + 8);
         hipLaunchKernelGGL(k_emit_tail, dim3(grid_for(tail, WG, 1024)), dim3(WG), 0, s, l, d_v, d_m,
-                           (const uint64_t *)start, (const uint32_t *)bws, out->meta, d_append,
+                           (const uint64_t *)start, (const uint32_t *)bws, out->meta,
                            f.kind == MS_DELTA ? out->refs : (uint64_t *)nullptr, out->data, (const uint64_t *)nullptr,
                            (const uint64_t *)nullptr);
     }
@@ -834,7 +1252,7 @@ int launch_emit_flags(ms_col *out, const sel_flags &sf, const sel_split &sp, uin
         return ms_fail(MS_ERR_CAPACITY, "emit: delta carries capacity");
     const uint64_t tail = std::max<uint64_t>(l.bs + l.K + 1, m_bound / MS_DELTA_TILE * 8 + 8);
     hipLaunchKernelGGL(k_emit_tail, dim3(grid_for(tail, WG, 1024)), dim3(WG), 0, s, l, (const uint64_t *)pos, d_m,
-                       (const uint64_t *)start, (const uint32_t *)bws, out->meta, (uint64_t *)nullptr,
+                       (const uint64_t *)start, (const uint32_t *)bws, out->meta,
                        f.kind == MS_DELTA ? out->refs : (uint64_t *)nullptr, out->data, d_total,
                        (const uint64_t *)sp.d_flag);
     MS_HIP(hipGetLastError());

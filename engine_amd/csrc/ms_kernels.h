@@ -37,6 +37,10 @@ int plan_hold(void (*release)(void *), void *obj);
 void *dev_alloc(size_t bytes, hipStream_t s);
 void dev_free(void *p, hipStream_t s);
 
+// Workgroups of `kernel` (wg threads, no dynamic LDS) that the current
+// device holds at once, queried once per kernel.
+uint32_t resident_grid(const void *kernel, uint32_t wg);
+
 // decode side -------------------------------------------------------
 int launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t s);
 // Caller-provided device buffers of launch_select_sum: `part` holds
@@ -85,10 +89,9 @@ int launch_exclusive_scan_n(const uint64_t *d_in, uint64_t *d_out, const uint64_
 // Emits the m values d_v[0 .. *d_m) into `out` (already allocated, format
 // out->f) as `chunk`-value morph_batch calls (chunk 0: one call for the
 // whole compressed part, i.e. a column-level morph) followed by the raw
-// rest, and sets out's meta.  *d_append receives the write-iterator's
-// append offset (done()'s second element).
-int launch_emit(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, uint64_t m_bound, uint64_t chunk,
-                uint64_t *d_append, temps &sc);
+// rest, and sets out's meta (which needs no clearing before; aux[0] is the
+// write-iterator's append offset, done()'s second element).
+int launch_emit(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, uint64_t m_bound, uint64_t chunk, temps &sc);
 // The select's split of its input (select_compr.h:209-250): rows below
 // the scalar remainder's first row go through the write-iterator, the
 // positions of the remainder's selected rows are appended raw behind it.

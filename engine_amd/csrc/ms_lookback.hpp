@@ -1,0 +1,86 @@
+// ms_lookback.hpp -- prefix sums over the tiles of one launch.
+//
+// A kernel whose output offsets depend on every tile before it takes its
+// tiles in ticket order and publishes one 64-bit word per tile: first the
+// tile's own total, then (once known) the total of all tiles up to it.  A
+// tile's offset is found by one wave reading 64 predecessors' words at a
+// time.  Progress: a tile's ticket is only handed out after every earlier
+// ticket, so each word that is waited for belongs to a workgroup that
+// already runs, and a tile publishes its total before it waits.
+// The words and the ticket counter are cleared before the launch.
+#pragma once
+
+#include "ms_device.hpp"
+
+namespace ms {
+
+constexpr uint64_t LB_TOTAL = 1ull << 62;      // the tile's own total
+constexpr uint64_t LB_PREFIX = 2ull << 62;     // the total up to and with the tile
+constexpr uint64_t LB_VALUE = LB_TOTAL - 1ull;
+
+__device__ __forceinline__ uint64_t lb_load(const uint64_t *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void lb_store(uint64_t *p, uint64_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The next ticket of a launch (one thread).
+__device__ __forceinline__ uint64_t lb_ticket(uint64_t *counter)
+{
+    return __hip_atomic_fetch_add(counter, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Publishes a tile's own total (below 2^62; one wave).
+__device__ __forceinline__ void lb_publish(uint64_t *words, uint64_t tile, uint64_t total)
+{
+    if (lane_id() == 0) lb_store(words + tile, (tile ? LB_TOTAL : LB_PREFIX) | total);
+}
+
+// Sum of the totals of tiles 0 .. tile - 1, after lb_publish of this tile's
+// `total`.  All 64 lanes of one wave call it.  A step reads the words of
+// LB_SPAN x 64 predecessors: a launch's first tiles publish at about the
+// same time, far from any prefix.
+constexpr uint32_t LB_SPAN = 2;
+
+__device__ __forceinline__ uint64_t lb_exclusive(uint64_t *words, uint64_t tile, uint64_t total)
+{
+    const uint32_t t = lane_id();
+    if (tile == 0) return 0;
+    uint64_t sum = 0;
+    int64_t last = (int64_t)tile - 1;          // the nearest word of the step: row 0, lane 0
+    for (;;) {
+        uint64_t w[LB_SPAN];
+#pragma unroll
+        for (uint32_t i = 0; i < LB_SPAN; i++) {
+            const int64_t k = last - (int64_t)(64 * i + t);
+            w[i] = k >= 0 ? lb_load(words + k) : LB_PREFIX;
+        }
+        bool found = false;
+#pragma unroll
+        for (uint32_t i = 0; i < LB_SPAN; i++) {
+            if (found) continue;
+            // wait for the row's words up to its nearest prefix
+            uint64_t pre;
+            for (;;) {
+                pre = __ballot((w[i] & LB_PREFIX) != 0);
+                const uint64_t none = __ballot(w[i] == 0);
+                if ((none & (pre ? (pre & (0ull - pre)) - 1ull : ~0ull)) == 0) break;
+                __builtin_amdgcn_s_sleep(1);
+                if (w[i] == 0) w[i] = lb_load(words + (last - (int64_t)(64 * i + t)));
+            }
+            const uint32_t stop = pre ? (uint32_t)__builtin_ctzll(pre) : 63u;
+            sum += t <= stop ? w[i] & LB_VALUE : 0ull;
+            found = pre != 0;
+        }
+        if (found) break;
+        last -= 64 * LB_SPAN;
+    }
+    sum = wave_sum_u64(sum);
+    if (t == 0) lb_store(words + tile, LB_PREFIX | (sum + total));
+    return sum;
+}
+
+}  // namespace ms
