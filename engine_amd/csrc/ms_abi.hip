@@ -1131,7 +1131,7 @@ extern "C" int ms_morph(ms_col **out, const ms_format_desc *dst, const ms_col *i
         return bwi_new(*dst, vals, n, nullptr, sc, out);
     }
     if (dst->kind == MS_RLE) {
-        MS_TRY(new_col(*dst, nb, 16 * nb + 64, S(stream), &c));
+        MS_TRY(new_col(*dst, nb, 16 * nb + 64, S(stream), &c, nullptr, false));
         int rc = launch_rle_compress(c, vals, d_n, nb, sc);
         if (rc) { ms_col_free(c); return rc; }
         *out = c;

@@ -40,24 +40,28 @@ __device__ __forceinline__ void lb_publish(uint64_t *words, uint64_t tile, uint6
 }
 
 // Sum of the totals of tiles 0 .. tile - 1, after lb_publish of this tile's
-// `total`.  All 64 lanes of one wave call it.  A step reads the words of
-// LB_SPAN x 64 predecessors: a launch's first tiles publish at about the
-// same time, far from any prefix.
+// `total`, in two halves (all 64 lanes of one wave): lb_request asks for
+// the words of the 64 LB_SPAN tiles in front, lb_exclusive waits for them.
+// Loads return in order, so what a wave loads between the two does not
+// delay its words; a step past them does wait for it.
 constexpr uint32_t LB_SPAN = 2;
 
-__device__ __forceinline__ uint64_t lb_exclusive(uint64_t *words, uint64_t tile, uint64_t total)
+__device__ __forceinline__ void lb_request(const uint64_t *words, int64_t last, uint64_t (&w)[LB_SPAN])
+{
+#pragma unroll
+    for (uint32_t i = 0; i < LB_SPAN; i++) {
+        const int64_t k = last - (int64_t)(64 * i + lane_id());
+        w[i] = k >= 0 ? lb_load(words + k) : LB_PREFIX;
+    }
+}
+
+__device__ __forceinline__ uint64_t lb_exclusive(uint64_t *words, uint64_t tile, uint64_t total,
+                                                 uint64_t (&w)[LB_SPAN])
 {
     const uint32_t t = lane_id();
     if (tile == 0) return 0;
     uint64_t sum = 0;
-    int64_t last = (int64_t)tile - 1;          // the nearest word of the step: row 0, lane 0
-    for (;;) {
-        uint64_t w[LB_SPAN];
-#pragma unroll
-        for (uint32_t i = 0; i < LB_SPAN; i++) {
-            const int64_t k = last - (int64_t)(64 * i + t);
-            w[i] = k >= 0 ? lb_load(words + k) : LB_PREFIX;
-        }
+    for (int64_t last = (int64_t)tile - 1;;) {   // the nearest word of the step: row 0, lane 0
         bool found = false;
 #pragma unroll
         for (uint32_t i = 0; i < LB_SPAN; i++) {
@@ -77,6 +81,7 @@ __device__ __forceinline__ uint64_t lb_exclusive(uint64_t *words, uint64_t tile,
         }
         if (found) break;
         last -= 64 * LB_SPAN;
+        lb_request(words, last, w);
     }
     sum = wave_sum_u64(sum);
     if (t == 0) lb_store(words + tile, LB_PREFIX | (sum + total));
