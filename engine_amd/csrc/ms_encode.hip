@@ -879,6 +879,7 @@ __global__ __launch_bounds__(OP_WAVES * 64, 4) void k_emit_onepass(emit_layout l
     const auto blocks_of = [&](uint64_t b0) -> uint32_t {    // blocks of a wave that starts at b0
         return b0 >= pl.nb ? 0u : pl.nb - b0 < OP_WB ? (uint32_t)(pl.nb - b0) : OP_WB;
     };
+    if (blockIdx.x >= ntiles) return;   // as many workgroups as tiles take tickets
     if (threadIdx.x == 0) s_tile = lb_ticket(state);
     __syncthreads();
     uint64_t tile = readlane64(s_tile, 0);   // uniform: addresses and branches stay scalar
@@ -1441,6 +1442,7 @@ __global__ __launch_bounds__(RLE_WAVES * 64, 4) void k_rle_onepass(const uint64_
     const auto values_of = [&](uint64_t i0) -> uint32_t {
         return i0 >= m ? 0u : m - i0 < RLE_WV ? (uint32_t)(m - i0) : RLE_WV;
     };
+    if (blockIdx.x >= ntiles) return;   // as many workgroups as tiles take tickets
     if (threadIdx.x == 0) s_tile = lb_ticket(state);
     __syncthreads();
     uint64_t tile = readlane64(s_tile, 0);
