@@ -1,7 +1,10 @@
 // ms_abi.hip -- the C-ABI of include/morphstore_hip.h: column management
 // and operator orchestration.  Entry points never throw; errors are status
 // codes with a per-thread message (ms_last_error).
+#include <list>
+#include <map>
 #include <mutex>
+#include <unordered_map>
 #include <unordered_set>
 #include <stdarg.h>
 #include <stdio.h>
@@ -62,6 +65,16 @@ static thread_local ms_plan *g_rec = nullptr;
 
 static uint64_t round256(uint64_t x) { return (x + 255) / 256 * 256; }
 
+// hipMalloc, with the kept memory of the null stream given back if it fails.
+static hipError_t malloc_arena(uint8_t **p, size_t bytes)
+{
+    hipError_t e = hipMalloc((void **)p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    ms::release_kept();
+    return hipMalloc((void **)p, bytes);
+}
+
 namespace ms {
 
 bool plan_capturing() { return g_rec && g_rec->recording && g_rec->mode == 1; }
@@ -71,6 +84,154 @@ int plan_hold(void (*release)(void *), void *obj)
     if (!plan_capturing()) return ms_fail(MS_ERR_INVALID, "no plan is capturing");
     g_rec->holds.emplace_back(release, obj);
     return MS_OK;
+}
+
+// ------------------------------------------------------------------
+// Memory of the null stream, kept for its next call.  hipMallocAsync's pool
+// gives memory back to the system on a free whatever its release threshold
+// says, so that every call maps and unmaps its buffers again: of the
+// select, project and agg_sum over 2^24 values (0.31 ms of kernels) that
+// was 0.8 to 12 ms, growing with the memory the process holds.  A block
+// freed on the null stream is handed to a later call on the null stream
+// without waiting: the stream orders its uses, and unlike a created
+// stream it is never destroyed and never captured; other streams keep
+// using hipMallocAsync.  At most a sixteenth of the device's memory is
+// kept (the least recently freed blocks go first), all of it is given back
+// when an allocation of the library fails and when the last column is freed.
+// ------------------------------------------------------------------
+namespace {
+
+struct null_cache {
+    struct block {
+        void *p;
+        size_t bytes;
+        int dev;
+    };
+    typedef std::list<block> lru;                       // free blocks, least recently freed first
+    std::mutex mu;
+    std::unordered_map<void *, block> live;             // blocks in use
+    lru free_;
+    std::map<std::pair<int, size_t>, std::vector<lru::iterator>> by_size;   // (device, bytes)
+    size_t kept = 0, limit = 0;
+
+    // Sizes are rounded so that calls of nearly the same sizes share
+    // blocks: eighths of a power of two, at most 32 MiB.
+    static size_t round_size(size_t n)
+    {
+        size_t step = 256;
+        while (step * 16 <= n && step < (32u << 20)) step *= 2;
+        return (n + step - 1) / step * step;
+    }
+
+    void unlink(lru::iterator it)
+    {
+        auto b = by_size.find({it->dev, it->bytes});
+        for (auto k = b->second.begin(); k != b->second.end(); ++k)
+            if (*k == it) {
+                b->second.erase(k);
+                break;
+            }
+        if (b->second.empty()) by_size.erase(b);
+        kept -= it->bytes;
+        free_.erase(it);
+    }
+
+    void trim(size_t to)
+    {
+        while (kept > to && !free_.empty()) {
+            void *p = free_.front().p;
+            unlink(free_.begin());
+            (void)hipFreeAsync(p, nullptr);
+        }
+    }
+
+    // Everything kept, to the system (waits for the device).
+    void give_back()
+    {
+        if (free_.empty()) return;
+        trim(0);
+        int dev = 0;
+        hipMemPool_t pool;
+        (void)hipDeviceSynchronize();
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
+            (void)hipMemPoolTrimTo(pool, 0);
+    }
+
+    void *get(size_t bytes)
+    {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+        const size_t want = round_size(bytes);
+        std::lock_guard<std::mutex> lk(mu);
+        // the smallest block that fits, unless it is much too large
+        auto b = by_size.lower_bound({dev, want});
+        if (b != by_size.end() && b->first.first == dev && b->first.second <= want + want / 4) {
+            const lru::iterator it = b->second.back();
+            const block k = *it;
+            unlink(it);
+            live[k.p] = k;
+            return k.p;
+        }
+        block k = {nullptr, want, dev};
+        if (hipMallocAsync(&k.p, want, nullptr) != hipSuccess) {
+            (void)hipGetLastError();
+            give_back();
+            k.bytes = bytes;
+            if (hipMallocAsync(&k.p, bytes, nullptr) != hipSuccess) return nullptr;
+        }
+        live[k.p] = k;
+        return k.p;
+    }
+
+    // false: not one of this cache's blocks
+    bool put(void *p)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto l = live.find(p);
+        if (l == live.end()) return false;
+        const block k = l->second;
+        live.erase(l);
+        if (!limit) {
+            size_t avail = 0, total = 0;
+            limit = hipMemGetInfo(&avail, &total) == hipSuccess && total ? total / 16 : 1u << 30;
+        }
+        if (k.bytes > limit) {
+            (void)hipFreeAsync(p, nullptr);
+            return true;
+        }
+        free_.push_back(k);
+        by_size[{k.dev, k.bytes}].push_back(std::prev(free_.end()));
+        kept += k.bytes;
+        trim(limit);
+        return true;
+    }
+
+
+    void drop()
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        trim(0);
+    }
+};
+
+null_cache &cache()
+{
+    static null_cache *c = new null_cache();   // outlives every static object's destructor
+    return *c;
+}
+
+}  // namespace
+
+void release_kept()
+{
+    std::lock_guard<std::mutex> lk(cache().mu);
+    cache().give_back();
+}
+
+// Frees memory of dev_alloc (or of a created stream) in order on s.
+static void free_ordered(void *p, hipStream_t s)
+{
+    if (!cache().put(p)) (void)hipFreeAsync(p, s);
 }
 
 void *dev_alloc(size_t bytes, hipStream_t s)
@@ -83,7 +244,13 @@ void *dev_alloc(size_t bytes, hipStream_t s)
         return p;
     }
     void *p = nullptr;
-    if (hipMallocAsync(&p, bytes, s) != hipSuccess) return nullptr;
+    if (s == nullptr) p = cache().get(bytes);
+    else if (hipMallocAsync(&p, bytes, s) != hipSuccess) {
+        (void)hipGetLastError();
+        release_kept();
+        if (hipMallocAsync(&p, bytes, s) != hipSuccess) return nullptr;
+    }
+    if (!p) return nullptr;
     if (g_rec && g_rec->recording && g_rec->mode == 0) g_rec->measured += bytes;
     return p;
 }
@@ -97,7 +264,7 @@ static bool in_arena(const void *p)
 void dev_free(void *p, hipStream_t s)
 {
     if (!p || in_arena(p)) return;
-    (void)hipFreeAsync(p, s);
+    free_ordered(p, s);
 }
 
 void *temps::get(size_t bytes)
@@ -666,16 +833,19 @@ extern "C" uint64_t ms_col_count_bound(const ms_col *c) { return c ? c->count_bo
 extern "C" int ms_col_free(ms_col *c)
 {
     if (!c) return MS_OK;
+    bool last;
     {
         std::lock_guard<std::mutex> lk(g_cols_mu);
         if (!g_cols.erase(c)) return ms_fail(MS_ERR_INVALID, "ms_col_free: not a live column handle");
+        last = g_cols.empty();
     }
     if (c->arena) {
         // arena columns die with their plan
     } else if (g_rec && g_rec->recording && g_rec->mode == 1) {
         g_rec->deferred.push_back((void *)c->meta);   // a free now would be captured into the graph
     } else {
-        (void)hipFreeAsync((void *)c->meta, c->stream);
+        free_ordered((void *)c->meta, c->stream);
+        if (last) cache().drop();
     }
     delete c->bwi;
     delete c;
@@ -830,7 +1000,7 @@ extern "C" int ms_plan_create(ms_plan **out, uint64_t arena_bytes)
     if (!p) return ms_fail(MS_ERR_NOMEM, "host allocation");
     p->arena_bytes = arena_bytes;
     p->mode = arena_bytes ? 1 : 0;
-    if (arena_bytes && hipMalloc((void **)&p->arena, arena_bytes) != hipSuccess) {
+    if (arena_bytes && malloc_arena(&p->arena, arena_bytes) != hipSuccess) {
         delete p;
         return ms_fail(MS_ERR_NOMEM, "plan arena of %llu bytes", (unsigned long long)arena_bytes);
     }
@@ -845,7 +1015,7 @@ extern "C" int ms_plan_begin(ms_plan *p, void *stream)
     if (p->mode == 0 && p->measured) {
         // the measuring pass is done: allocate the arena and capture
         p->arena_bytes = p->measured + (1u << 20);
-        if (hipMalloc((void **)&p->arena, p->arena_bytes) != hipSuccess)
+        if (malloc_arena(&p->arena, p->arena_bytes) != hipSuccess)
             return ms_fail(MS_ERR_NOMEM, "plan arena of %llu bytes", (unsigned long long)p->arena_bytes);
         p->mode = 1;
     }
@@ -876,7 +1046,7 @@ extern "C" int ms_plan_end(ms_plan *p, void *stream)
         return MS_OK;
     }
     hipError_t e = hipStreamEndCapture(p->stream, &p->graph);
-    for (void *q : p->deferred) (void)hipFreeAsync(q, p->stream);
+    for (void *q : p->deferred) free_ordered(q, p->stream);
     p->deferred.clear();
     if (e != hipSuccess) return ms_fail(MS_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
     MS_HIP(hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0));

@@ -409,7 +409,12 @@ static int ensure(T **p, size_t &cap, size_t n)
     if (*p) MS_HIP(hipFree(*p));
     *p = nullptr;
     cap = 0;
-    MS_HIP(hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T)));
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+    if (hipMalloc((void **)p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        release_kept();
+        MS_HIP(hipMalloc((void **)p, bytes));
+    }
     cap = std::max<size_t>(n, 1);
     return MS_OK;
 }

@@ -36,6 +36,9 @@ int plan_hold(void (*release)(void *), void *obj);
 // device memory of the operators (from a recording plan's arena if any)
 void *dev_alloc(size_t bytes, hipStream_t s);
 void dev_free(void *p, hipStream_t s);
+// gives back the memory that dev_alloc keeps for the null stream (for a
+// direct allocation that failed; waits for the device)
+void release_kept();
 
 // Workgroups of `kernel` (wg threads, no dynamic LDS) that the current
 // device holds at once, queried once per kernel.

@@ -1,0 +1,75 @@
+"""Memory of the null stream is kept for its next calls: blocks that go from
+one call's output to another's scratch, columns read on a created stream
+before they are freed, frees from several threads, and frees while a plan
+captures leave every result as it was."""
+import threading
+
+import numpy as np
+import pytest
+
+import engine_amd as ea
+from engine_amd import datagen, hip
+from engine_amd.formats import MS_CMP_LT, default_delta_dynamic_vbp_f, dynamic_vbp_f, rle_f, uncompr_f
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    ea.init(0)
+
+
+def below(x, v):
+    return int(x[x < v].sum(dtype=np.uint64))
+
+
+def test_columns_read_on_a_created_stream():
+    st, res = hip.Stream(), ea.DeviceU64(40)
+    want = []
+    for k in range(40):
+        x = datagen.uniform_bits(100 + k, 30_000 + 512 * (k % 3), 20)
+        col = ea.morph(dynamic_vbp_f(512, 2048, 8), ea.upload_values(x))
+        ea.select_sum(MS_CMP_LT, 1 << 19, col, res.at(k), st)
+        want.append(below(x, 1 << 19))
+        del col         # its block serves the next column while the stream still reads it
+    assert res.get().tolist() == want
+
+
+def test_threads_share_the_null_stream():
+    bad = []
+
+    def work(seed):
+        ea.init(0)
+        for k in range(12):
+            n = 5000 + 7001 * (k % 4) + seed
+            x = datagen.sorted_geometric(seed + k, n)
+            f = (default_delta_dynamic_vbp_f(8), rle_f(), dynamic_vbp_f(512, 64, 8))[k % 3]
+            c = ea.morph(f, ea.upload_values(x))
+            if not np.array_equal(ea.morph(uncompr_f(), c).values(), x):
+                bad.append((seed, k))
+
+    ts = [threading.Thread(target=work, args=(1000 * i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad
+
+
+def test_free_while_a_plan_captures():
+    st, plan = hip.Stream(), ea.Plan()
+    x = datagen.uniform_bits(3, 50_000, 16)
+    col = ea.morph(dynamic_vbp_f(512, 2048, 8), ea.upload_values(x))
+    hip.synchronize()
+    spare = ea.upload_values(x)
+    with plan.record(st):
+        ea.agg_sum(col, st)
+    with plan.record(st):
+        total = ea.agg_sum(col, st)
+        del spare       # given back at the end of the capture
+    again = ea.upload_values(x ^ np.uint64(1))
+    for _ in range(3):
+        plan.launch(st)
+        st.synchronize()
+        assert int(total.values(st)[0]) == int(x.sum(dtype=np.uint64))
+        assert np.array_equal(again.values(), x ^ np.uint64(1))
+    del total
+    plan.free()
