@@ -1355,10 +1355,22 @@ static int select_pred(ms_col **out, const ms_pred &p, const ms_format_desc *out
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
     temps sc(S(stream));
     const uint64_t nb = in->count_bound;
-    uint64_t *pos = (uint64_t *)sc.get(nb * 8 + 64);
     uint64_t *d = (uint64_t *)sc.get(64);
-    if (!pos || !d) return ms_fail(MS_ERR_NOMEM, "select scratch");
+    if (!d) return ms_fail(MS_ERR_NOMEM, "select scratch");
     uint64_t *d_cnt = d, *d_na = d + 1, *d_flag = d + 2;
+    if (out_f->kind == MS_UNCOMPR) {
+        // the write-iterator's values and the raw append behind them are
+        // one array: the positions go straight into the column
+        ms_col *c;
+        MS_TRY(new_col(*out_f, nb + 64, out_capacity(*out_f, nb + 64, wit_chunk(*out_f)), S(stream), &c, nullptr,
+                       false));
+        const int rc = launch_select_positions(in, p, (uint64_t *)c->data, d_cnt, sc, c->meta);
+        if (rc) { ms_col_free(c); return rc; }
+        *out = c;
+        return MS_OK;
+    }
+    uint64_t *pos = (uint64_t *)sc.get(nb * 8 + 64);
+    if (!pos) return ms_fail(MS_ERR_NOMEM, "select scratch");
     if (select_flags_ok(in) && emit_flags_ok(*out_f)) {
         // positions go from the count pass's ballots straight into the
         // output format; pos only receives the few read by rank
@@ -1458,6 +1470,16 @@ extern "C" int ms_project(ms_col **out, const ms_format_desc *out_f, const ms_co
         tmpdata.count_bound = data->count_bound;
         dsrc = &tmpdata;
     }
+    if (out_f->kind == MS_UNCOMPR) {
+        // the write-iterator's values and the raw append behind them are
+        // one array: the values go straight into the column
+        ms_col *c;
+        MS_TRY(new_col(*out_f, np + 64, out_capacity(*out_f, np + 64, wit_chunk(*out_f)), S(stream), &c));
+        const int rc = launch_gather(dsrc, pv, d_np, np, (uint64_t *)c->data, &c->meta->status, sc, c->meta);
+        if (rc) { ms_col_free(c); return rc; }
+        *out = c;
+        return MS_OK;
+    }
     uint64_t *v = (uint64_t *)sc.get(np * 8 + 64);
     uint64_t *d = (uint64_t *)sc.get(64);
     if (!v || !d) return ms_fail(MS_ERR_NOMEM, "project scratch");
@@ -1477,26 +1499,16 @@ extern "C" int ms_project(ms_col **out, const ms_format_desc *out_f, const ms_co
 }
 
 // ------------------------------------------------------------------ agg_sum
-__global__ void k_agg_meta(ms_dev_meta *m, uint64_t compr)
-{
-    m->count = 1;
-    m->size_used = 8;
-    m->size_compr = compr;
-}
-
 extern "C" int ms_agg_sum(ms_col **out, const ms_col *in, void *stream)
 {
     MS_TRY(ms_need_init());
     if (!out || !in) return ms_fail(MS_ERR_INVALID, "bad argument");
     ms_col *c;
-    MS_TRY(new_col(uncompr_desc(), 1, 64, S(stream), &c));
+    MS_TRY(new_col(uncompr_desc(), 1, 64, S(stream), &c, nullptr, false));
     ms_pred all = make_pred(MS_CMP_GE, 0);
-    int rc = launch_select_sum(in, all, (uint64_t *)c->data, false, S(stream));
-    if (!rc) {
-        // agg_sum_compr.h:148-150 vs agg_sum_uncompr.h:126 (sizeCompr 8 vs 0)
-        hipLaunchKernelGGL(k_agg_meta, dim3(1), dim3(1), 0, S(stream), c->meta, in->f.kind == MS_UNCOMPR ? 0ull : 8ull);
-        if (hipGetLastError() != hipSuccess) rc = ms_fail(MS_ERR_HIP, "agg_sum meta");
-    }
+    // agg_sum_compr.h:148-150 vs agg_sum_uncompr.h:126 (sizeCompr 8 vs 0)
+    const int rc = launch_select_sum(in, all, (uint64_t *)c->data, false, S(stream), nullptr, c->meta,
+                                     in->f.kind == MS_UNCOMPR ? 0ull : 8ull);
     if (rc) { ms_col_free(c); return rc; }
     *out = c;
     return MS_OK;

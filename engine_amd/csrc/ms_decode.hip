@@ -682,53 +682,6 @@ __global__ __launch_bounds__(WG) void k_rle_expand(ms_colv c, const uint64_t *cs
 }
 
 // ------------------------------------------------------------------
-// Select positions over uncompressed values: per 512-value unit a count,
-// an exclusive scan, then compaction in index order (value i of a unit is
-// u*512 + 64m + t, so ballots in m order give ascending ranks).
-// ------------------------------------------------------------------
-__global__ __launch_bounds__(WG) void k_sel_count(const uint64_t *x, const uint64_t *d_n, ms_pred p, uint64_t *cnt,
-                                                   uint64_t units_bound)
-{
-    const uint64_t n = *d_n;
-    const uint32_t t = threadIdx.x & 63;
-    const uint64_t nwaves = (uint64_t)gridDim.x * WAVES;
-    for (uint64_t u = (uint64_t)blockIdx.x * WAVES + wave_index(); u < units_bound; u += nwaves) {
-        uint32_t c = 0;
-#pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const uint64_t i = u * 512 + 64 * m + t;
-            const bool take = i < n && pred_eval(p, x[i]);
-            c += __popcll(__ballot(take));
-        }
-        if (t == 0) cnt[u] = c;
-    }
-}
-
-__global__ __launch_bounds__(WG) void k_sel_compact(const uint64_t *x, const uint64_t *d_n, ms_pred p,
-                                                     const uint64_t *off, uint64_t *pos, uint64_t units_bound,
-                                                     uint64_t *d_cnt)
-{
-    const uint64_t n = *d_n;
-    const uint32_t t = threadIdx.x & 63;
-    const uint64_t nwaves = (uint64_t)gridDim.x * WAVES;
-    const uint64_t nunits = (n + 511) / 512;
-    for (uint64_t u = (uint64_t)blockIdx.x * WAVES + wave_index(); u < nunits; u += nwaves) {
-        uint64_t o = off[u];
-#pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const uint64_t i = u * 512 + 64 * m + t;
-            const bool take = i < n && pred_eval(p, x[i]);
-            const uint64_t bal = __ballot(take);
-            if (take) pos[o + __popcll(bal & ((1ull << t) - 1ull))] = i;
-            o += __popcll(bal);
-        }
-        if (u == nunits - 1 && t == 0) *d_cnt = o;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0 && n == 0) *d_cnt = 0;
-    (void)units_bound;
-}
-
-// ------------------------------------------------------------------
 // Host launchers
 // ------------------------------------------------------------------
 static bool fast_blocks(const ms_colv &v)
@@ -771,11 +724,22 @@ static static_dec_t static_dec_kernel(uint32_t bw)
     }
 }
 
+// The meta of a column of one uncompressed value (an aggregate's result).
+__device__ __forceinline__ void set_meta_one(ms_dev_meta *om, uint64_t compr)
+{
+    om->count = 1;
+    om->size_used = 8;
+    om->size_compr = compr;
+    om->status = 0;
+    for (int k = 0; k < 4; k++) om->aux[k] = 0;
+}
+__global__ void k_set_meta_one(ms_dev_meta *om, uint64_t compr) { set_meta_one(om, compr); }
+
 // Sums the per-workgroup partials and the uncompressed rest (select + sum
 // over the rest part, the vectorised and scalar loops of
 // agg_sum_compr.h:110-146 folded into one) and writes the result.
 __global__ __launch_bounds__(WG) void k_sum_finish(ms_colv c, ms_pred p, const uint64_t *part, uint32_t nparts,
-                                                   int with_rest, uint64_t *result)
+                                                   int with_rest, uint64_t *result, ms_dev_meta *om, uint64_t om_compr)
 {
     uint64_t acc = 0;
     for (uint32_t i = threadIdx.x; i < nparts; i += WG) acc += part[i];
@@ -792,6 +756,7 @@ __global__ __launch_bounds__(WG) void k_sum_finish(ms_colv c, ms_pred p, const u
         uint64_t sum = 0;
         for (int w = 0; w < WAVES; w++) sum += s_part[w];
         *result = sum;
+        if (om) set_meta_one(om, om_compr);
     }
 }
 
@@ -875,13 +840,16 @@ static uint32_t stride_grid(const void *kernel, uint64_t items)
 }
 
 int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bool accumulate, hipStream_t s,
-                      const ss_buffers *bufs)
+                      const ss_buffers *bufs, ms_dev_meta *om, uint64_t om_compr)
 {
     ms_colv v;
     MS_TRY(colv_of(in, v));
     if (v.g.kind == MS_BLOCKWISE_INDIVIDUAL) {
         if (bufs) return ms_fail(MS_ERR_INVALID, "blockwise_individual_f: select_sum needs temporaries of its own");
-        return launch_bwi_select_sum(in, p, d_result, accumulate, s);
+        MS_TRY(launch_bwi_select_sum(in, p, d_result, accumulate, s));
+        if (om) hipLaunchKernelGGL(k_set_meta_one, dim3(1), dim3(1), 0, s, om, om_compr);
+        MS_HIP(hipGetLastError());
+        return MS_OK;
     }
     temps sc(s);
     const uint64_t nb = in->count_bound;
@@ -963,7 +931,8 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
     }
     MS_HIP(hipGetLastError());
     static_assert(SS_MAX_PARTS >= 8192, "every grid above is capped at 8192 workgroups");
-    hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(WG), 0, s, v, p, (const uint64_t *)part, grid, with_rest, d_result);
+    hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(WG), 0, s, v, p, (const uint64_t *)part, grid, with_rest, d_result,
+                       om, om_compr);
     MS_HIP(hipGetLastError());
     return MS_OK;
 }
@@ -1072,10 +1041,6 @@ int launch_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s, ms_dev_m
     return MS_OK;
 }
 
-__global__ void k_count_of(const ms_dev_meta *m, uint64_t *dst) { *dst = m->count; }
-
-__global__ void k_units_of(const ms_dev_meta *m, uint64_t *dst) { *dst = (m->count + 511) / 512; }
-
 // Flags of unit u's 512 values (bit t of the result's word m = value
 // 64 * (t >> 3) + 8 * m + (t & 7) of the unit, lane-major per thread):
 // decoded from the compressed part, or read raw from the rest.
@@ -1084,7 +1049,9 @@ __global__ void k_units_of(const ms_dev_meta *m, uint64_t *dst) { *dst = (m->cou
 __device__ __forceinline__ void unit_entry(const ms_colv &c, uint64_t ncu, uint64_t u, uint64_t &e, uint64_t &r)
 {
     e = r = 0;
-    if (u < ncu) {
+    if (u < ncu && c.g.kind == MS_STATIC_VBP) {   // 8 lanes: 64 bw bytes per unit, no index
+        e = ((u * 64 * c.g.bw) << 8) | c.g.bw;
+    } else if (u < ncu) {
         const uint64_t b = u >> c.g.lg_spb;
         e = gload(c.index + b);
         if (c.g.kind == MS_FOR) r = gload(c.refs + (b >> c.g.lg_ipo));
@@ -1158,42 +1125,172 @@ __global__ __launch_bounds__(WG) void k_sel_count_blocks(ms_colv c, ms_pred p, u
     }
 }
 
-// Writes the selected positions of every unit from its stored ballots
-// (no second decode).
-__global__ __launch_bounds__(WG) void k_sel_compact_blocks(const uint64_t *flags, const uint64_t *d_units,
-                                                           const uint64_t *off, uint64_t *pos, uint64_t *d_cnt)
+// ------------------------------------------------------------------
+// Select positions: one pass over the rows, a wave per 1, 2 or 4 units of
+// 512 rows (per_wave), a workgroup's units one tile of a look-back over the
+// tiles' counts.
+// A unit's flags go to LDS as a bit per row (row r's 64 bits in word r); the
+// positions are written a tile later, when the tile's first rank is known
+// (its look-back then waits for no straggler).  Codes are tested as they are
+// decoded, so a bit-packed column is never expanded: SEL_LANES8 takes the
+// 8-lane indexed layouts and static_vbp_f<vbp_l<bw, 8>>, SEL_LANES1
+// static_vbp_f<vbp_l<bw, 1>>, SEL_RAW values (decompressed by the caller for
+// every other format).
+// Bound by the positions' stores and the tiles' tickets (about 20 ns each,
+// one counter for all XCDs).  Measured over 2^24 values of 12 bits, half of
+// them selected: 34 us from static_vbp_f<vbp_l<12, 1>> (decompression,
+// count, two scan kernels, compaction, split, copy and append before:
+// 200 us), 36 us from dynamic_vbp_f, 42 us from uncompr_f.
+// ------------------------------------------------------------------
+enum { SEL_LANES8 = 0, SEL_LANES1 = 1, SEL_RAW = 2 };
+constexpr uint32_t SEL_WAVES = 16, SEL_UNITS = 4;          // waves per tile, units per wave at most
+
+template <int SRC>
+__global__ __launch_bounds__(SEL_WAVES * 64) void k_select_onepass(ms_colv c, const uint64_t *x, ms_pred p,
+                                                                   uint64_t *state, uint64_t *pos, uint64_t *d_cnt,
+                                                                   ms_dev_meta *om, uint32_t per_wave)
 {
-    const uint64_t nunits = *d_units;
-    const uint32_t t = threadIdx.x & 63;
-    const uint64_t W = (uint64_t)gridDim.x * WAVES;
-    const uint64_t below = t ? (~0ull >> (64 - t)) : 0ull;
-    uint64_t u = (uint64_t)blockIdx.x * WAVES + wave_index();
-    // One load per lane requests a unit: lanes 0..7 its ballots, lane 8 its
-    // output offset (the other lanes re-read ballot 0).  The next unit is
-    // requested one unit ahead; past the end the current unit again.
-    const auto request = [&](uint64_t uu) {
-        return gload(t < 8 ? flags + 8 * uu + t : (t == 8 ? off + uu : flags + 8 * uu));
-    };
-    uint64_t my_n = u < nunits ? request(u) : 0ull;
-    for (; u < nunits; u += W) {
-        const uint64_t my = my_n;
-        my_n = request(u + W < nunits ? u + W : u);
-        // value 64 r + t of the unit is bit 8 r + (t & 7) of ballot t / 8:
-        // lane t takes that ballot, and row r's flags are one ballot of its
-        // bit r (a transpose of the 8 x 8 byte matrix, one step per row)
-        const uint64_t mine = __shfl(my, (int)(t >> 3), MS_WAVE);
-        uint64_t o = ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(my >> 32), 8) << 32) |
-                     __builtin_amdgcn_readlane((uint32_t)my, 8);
+    __shared__ uint64_t s_rows[2][SEL_WAVES][SEL_UNITS][8], s_ticket, s_base;
+    __shared__ uint32_t s_cnt[SEL_WAVES];
+    const ms_parts pt = parts_of(c);
+    const uint64_t nunits = (pt.n + 511) / 512, ncu = pt.n_compr >> 9;
+    const uint32_t tile_units = SEL_WAVES * per_wave;
+    const uint64_t ntiles = nunits ? (nunits + tile_units - 1) / tile_units : 1;
+    const uint32_t t = threadIdx.x & 63, w = wave_index();
+    uint64_t *tiles = state + 1;
+    if (blockIdx.x >= ntiles) return;   // as many workgroups as tiles take tickets
+    if (threadIdx.x == 0) s_ticket = lb_ticket(state);
+    __syncthreads();
+    uint64_t tile = readlane64(s_ticket, 0);
+    __syncthreads();
+    if (tile >= ntiles) return;
+    uint64_t ptile = ~0ull;                 // the tile that waits for its first rank
+    uint32_t pmine = 0, ptotal = 0;         // its rows of the waves before this one, of all
+    for (uint32_t turn = 0;; turn ^= 1) {
+        const bool have = tile < ntiles;
+        uint32_t n = 0;
+        if (have) {
+            if (threadIdx.x == 0) s_ticket = lb_ticket(state);
+            const uint64_t u0 = tile * tile_units + w * per_wave;
+            uint64_t my_e = 0, my_r = 0;    // lanes 0..3: the units' index entries and references
+            if (SRC == SEL_LANES8 && t < per_wave) unit_entry(c, ncu, u0 + t, my_e, my_r);
+#pragma unroll 1
+            for (uint32_t k = 0; k < per_wave; k++) {
+                const uint64_t u = u0 + k;
+                uint64_t *rows = s_rows[turn][w][k];
+                if (u >= nunits) {
+                    if (t < 8) rows[t] = 0;
+                    continue;
+                }
+                if (SRC == SEL_LANES8) {
+                    uint64_t B[8];
+                    unit_flags(c, pt, p, u, readlane64(my_e, k), readlane64(my_r, k), t, B);
+                    // byte gl of ballot m holds rows 64 gl + 8 m ..: byte m of row word gl
+                    uint64_t mine = B[0];
 #pragma unroll
-        for (uint32_t r = 0; r < 8; r++) {
-            const bool take = (mine >> (8 * r + (t & 7))) & 1;
-            const uint64_t F = __ballot(take);
-            if (take) pos[o + __popcll(F & below)] = u * 512 + 64 * r + t;
-            o += __popcll(F);
+                    for (uint32_t m = 0; m < 8; m++) {
+                        n += (uint32_t)__popcll(B[m]);
+                        if (m && (t >> 3) == m) mine = B[m];
+                    }
+                    ((uint8_t *)rows)[8 * (t & 7) + (t >> 3)] = (uint8_t)(mine >> (8 * (t & 7)));
+                } else if (SRC == SEL_LANES1) {
+                    // thread t holds rows 8 t .. 8 t + 7: wholly packed or wholly raw
+                    // (the packed part is a multiple of 64)
+                    uint64_t d[8];
+                    const uint64_t r0 = u * 512 + 8 * t;
+                    uint32_t in = 0xff;
+                    if (r0 < pt.n_compr) {
+                        uint64_t g = u * 64 + t;
+                        asm volatile("" : "+v"(g));   // keeps per-width offsets of g from being hoisted
+                        dec_dispatch(c.g.bw, (const uint64_t *)c.data, 1, 0, g, d);
+                    } else {
+                        const uint64_t *y = (const uint64_t *)(c.data + pt.rest_off) + (r0 - pt.n_compr);
+                        in = 0;
+#pragma unroll
+                        for (uint32_t m = 0; m < 8; m++) {
+                            const bool ok = r0 + m < pt.n;
+                            d[m] = ok ? gload(y + m) : 0ull;
+                            in |= ok ? 1u << m : 0u;
+                        }
+                    }
+                    uint32_t bits = 0;
+#pragma unroll
+                    for (uint32_t m = 0; m < 8; m++) {
+                        const bool take = ((in >> m) & 1) && pred_eval(p, d[m]);
+                        bits |= take ? 1u << m : 0u;
+                        n += (uint32_t)__popcll(__ballot(take));
+                    }
+                    ((uint8_t *)rows)[t] = (uint8_t)bits;
+                } else {
+                    uint64_t d[8], mine = 0;
+#pragma unroll
+                    for (uint32_t r = 0; r < 8; r++) {
+                        const uint64_t i = u * 512 + 64 * r + t;
+                        d[r] = i < pt.n ? gload(x + i) : 0ull;
+                    }
+#pragma unroll
+                    for (uint32_t r = 0; r < 8; r++) {
+                        const uint64_t F = __ballot(u * 512 + 64 * r + t < pt.n && pred_eval(p, d[r]));
+                        n += (uint32_t)__popcll(F);
+                        if (t == r) mine = F;
+                    }
+                    if (t < 8) rows[t] = mine;
+                }
+            }
+            if (t == 0) s_cnt[w] = n;
         }
-        if (u == nunits - 1 && t == 0) *d_cnt = o;
+        __syncthreads();
+        uint64_t next = ~0ull;
+        uint32_t mine = 0, total = 0;
+        if (have) {
+            next = readlane64(s_ticket, 0);
+#pragma unroll
+            for (uint32_t i = 0; i < SEL_WAVES; i++) {
+                if (i == w) mine = total;
+                total += __builtin_amdgcn_readfirstlane(s_cnt[i]);
+            }
+            if (w == 0) lb_publish(tiles, tile, total);
+        }
+        if (w == 0 && ptile != ~0ull) {
+            uint64_t words[LB_SPAN];
+            lb_request(tiles, (int64_t)ptile - 1, words);
+            const uint64_t base = lb_exclusive(tiles, ptile, ptotal, words);
+            if (t == 0) s_base = base;
+        }
+        __syncthreads();
+        if (ptile != ~0ull) {
+            uint64_t o = readlane64(s_base, 0) + pmine;
+            const uint64_t u0 = ptile * tile_units + w * per_wave;
+            // the wave's row words, one per lane
+            const uint64_t mine_w = (&s_rows[turn ^ 1][w][0][0])[t % (8 * SEL_UNITS)];
+#pragma unroll 4
+            for (uint32_t r = 0; r < 8 * per_wave; r++) {
+                const uint64_t F = readlane64(mine_w, r);
+                if (F == 0) continue;
+                if (__builtin_amdgcn_inverse_ballot_w64(F))
+                    pos[o + __builtin_amdgcn_mbcnt_hi((uint32_t)(F >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)F, 0))] =
+                        u0 * 512 + 64 * r + t;
+                o += (uint32_t)__popcll(F);
+            }
+            if (ptile == ntiles - 1 && threadIdx.x == 0) {
+                const uint64_t all = s_base + ptotal;
+                *d_cnt = all;
+                if (om) {
+                    om->count = all;
+                    om->size_used = 8 * all;
+                    om->size_compr = 0;
+                    om->status = 0;
+                    om->aux[0] = 8 * all;
+                    for (int k = 1; k < 4; k++) om->aux[k] = 0;
+                }
+            }
+        }
+        if (!have) return;
+        pmine = mine;
+        ptotal = total;
+        ptile = tile;
+        tile = next;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0 && nunits == 0) *d_cnt = 0;
 }
 
 bool select_flags_ok(const ms_col *in)
@@ -1229,52 +1326,39 @@ int launch_select_flags(const ms_col *in, const ms_pred &p, sel_flags &sf, temps
     return MS_OK;
 }
 
-int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos, uint64_t *d_cnt, temps &sc)
+int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos, uint64_t *d_cnt, temps &sc,
+                            ms_dev_meta *om)
 {
     hipStream_t s = sc.s;
     const uint64_t nb = in->count_bound;
     ms_colv v;
     MS_TRY(colv_of(in, v));
-    if ((v.g.kind == MS_DYNAMIC_VBP || v.g.kind == MS_FOR) && fast_blocks(v)) {
-        // decode, test and compact straight from the compressed units
-        const uint64_t units = nb / 512 + 1;
-        uint64_t *d_u = (uint64_t *)sc.get(64);
-        uint64_t *cnt = (uint64_t *)sc.get(units * 8 + 64);
-        uint64_t *off = (uint64_t *)sc.get(units * 8 + 64);
-        uint64_t *flags = (uint64_t *)sc.get(units * 64 + 64);
-        if (!d_u || !cnt || !off || !flags) return ms_fail(MS_ERR_NOMEM, "select scratch");
-        const dim3 grid(units_grid(nb));
-        hipLaunchKernelGGL(k_sel_count_blocks, grid, dim3(WG), 0, s, v, p, d_u, cnt, flags);
-        MS_HIP(hipGetLastError());
-        MS_TRY(launch_exclusive_scan_n(cnt, off, d_u, 0, units, sc));
-        hipLaunchKernelGGL(k_sel_compact_blocks, grid, dim3(WG), 0, s, (const uint64_t *)flags,
-                           (const uint64_t *)d_u, (const uint64_t *)off, d_pos, d_cnt);
-        MS_HIP(hipGetLastError());
-        return MS_OK;
-    }
-    const uint64_t *x;
-    if (in->g.kind == MS_UNCOMPR) {
+    // few units per wave while that leaves CUs without a tile, many for few
+    // tickets (2^18 rows: 8.1 / 9.3 / 13.4 us with 1 / 2 / 4 units, 2^24
+    // rows: 47 / 39 / 34 us)
+    const uint32_t per_wave = nb <= 1ull << 21 ? 1 : nb <= 1ull << 23 ? 2 : SEL_UNITS;
+    const uint64_t tiles = nb / (512ull * SEL_WAVES * per_wave) + 1;
+    uint64_t *state = (uint64_t *)sc.get((1 + tiles) * 8);
+    if (!state) return ms_fail(MS_ERR_NOMEM, "select scratch");
+    MS_TRY(launch_fill_u64(state, 1 + tiles, 0, s));
+    const bool lanes8 = ((v.g.kind == MS_DYNAMIC_VBP || v.g.kind == MS_FOR) && fast_blocks(v)) ||
+                        (v.g.kind == MS_STATIC_VBP && v.g.lanes == 8);
+    auto k = lanes8                                             ? k_select_onepass<SEL_LANES8>
+           : v.g.kind == MS_STATIC_VBP && v.g.lanes == 1        ? k_select_onepass<SEL_LANES1>
+                                                                : k_select_onepass<SEL_RAW>;
+    const uint64_t *x = nullptr;
+    if (k == k_select_onepass<SEL_RAW>) {
         x = (const uint64_t *)in->data;
-    } else {
-        uint64_t *tmp = (uint64_t *)sc.get(nb * 8 + 64);
-        if (!tmp) return ms_fail(MS_ERR_NOMEM, "select scratch");
-        MS_TRY(launch_decompress(in, tmp, s));
-        x = tmp;
+        if (in->g.kind != MS_UNCOMPR) {
+            uint64_t *tmp = (uint64_t *)sc.get(nb * 8 + 64);
+            if (!tmp) return ms_fail(MS_ERR_NOMEM, "select scratch");
+            MS_TRY(launch_decompress(in, tmp, s));
+            x = tmp;
+        }
     }
-    uint64_t *d_n = (uint64_t *)sc.get(64);
-    const uint64_t units = nb / 512 + 1;
-    uint64_t *cnt = (uint64_t *)sc.get(units * 8 + 64);
-    uint64_t *off = (uint64_t *)sc.get(units * 8 + 64);
-    if (!d_n || !cnt || !off) return ms_fail(MS_ERR_NOMEM, "select scratch");
-    uint64_t *d_u = (uint64_t *)sc.get(64);
-    if (!d_u) return ms_fail(MS_ERR_NOMEM, "select scratch");
-    hipLaunchKernelGGL(k_count_of, dim3(1), dim3(1), 0, s, in->meta, d_n);
-    hipLaunchKernelGGL(k_units_of, dim3(1), dim3(1), 0, s, in->meta, d_u);
-    hipLaunchKernelGGL(k_sel_count, dim3(grid_for(units, WAVES * 2ull)), dim3(WG), 0, s, x, d_n, p, cnt, units);
-    MS_HIP(hipGetLastError());
-    MS_TRY(launch_exclusive_scan_n(cnt, off, d_u, 0, units, sc));
-    hipLaunchKernelGGL(k_sel_compact, dim3(grid_for(units, WAVES * 2ull)), dim3(WG), 0, s, x, d_n, p, off, d_pos,
-                       units, d_cnt);
+    const uint32_t r = resident_grid((const void *)k, SEL_WAVES * 64);
+    hipLaunchKernelGGL(k, dim3(grid_for(tiles, 1, r)), dim3(SEL_WAVES * 64), 0, s, v, x, p, state, d_pos, d_cnt, om,
+                       per_wave);
     MS_HIP(hipGetLastError());
     return MS_OK;
 }

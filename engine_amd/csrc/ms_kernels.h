@@ -58,14 +58,18 @@ struct ss_buffers {
 };
 // *d_result (+)= sum of x_i with pred(x_i); the result is zeroed first
 // unless `accumulate`.  With `bufs` no device memory is allocated.
+// With `om` the result also sets the meta of the uncompr_f column d_result
+// is the one value of (count 1, `om_compr` compressed bytes).
 int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bool accumulate, hipStream_t s,
-                      const ss_buffers *bufs = nullptr);
+                      const ss_buffers *bufs = nullptr, ms_dev_meta *om = nullptr, uint64_t om_compr = 0);
 // writes the column's `count` values to d_out (uncompressed); with `om`
 // also the whole meta of the uncompr_f column d_out belongs to
 int launch_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s, ms_dev_meta *om = nullptr);
 // ascending positions with pred into d_pos (capacity >= count bound);
-// *d_cnt receives their number
-int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos, uint64_t *d_cnt, temps &sc);
+// *d_cnt receives their number; with `om` also the whole meta of the
+// uncompr_f column d_pos belongs to
+int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos, uint64_t *d_cnt, temps &sc,
+                            ms_dev_meta *om = nullptr);
 // The selected rows of a select as its count pass leaves them, without
 // materialising positions: 8 ballots per 512-row unit (bit 8 gl + j of
 // ballot m = row 64 gl + 8 m + j of the unit) and uoff[u] = the number of
@@ -199,8 +203,9 @@ int launch_xfmt_compress(ms_col *out, const uint64_t *d_v, const uint64_t *d_m, 
 int launch_xfmt_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s);
 
 // operators ---------------------------------------------------------
+// with `om` also the count and sizes of the uncompr_f column d_out belongs to
 int launch_gather(const ms_col *data, const uint64_t *d_pos, const uint64_t *d_np, uint64_t np_bound,
-                  uint64_t *d_out, uint64_t *d_status, temps &sc);
+                  uint64_t *d_out, uint64_t *d_status, temps &sc, ms_dev_meta *om = nullptr);
 int launch_intersect(const uint64_t *a, const uint64_t *d_na, uint64_t na_bound, const uint64_t *b,
                      const uint64_t *d_nb, uint64_t nb_bound, uint64_t *d_out, uint64_t *d_cnt, temps &sc);
 int launch_merge(const uint64_t *a, const uint64_t *d_na, uint64_t na_bound, const uint64_t *b,

@@ -63,10 +63,14 @@ __device__ __forceinline__ uint64_t gather_one(const ms_colv &c, const ms_parts 
 }
 
 __global__ __launch_bounds__(WG) void k_gather(ms_colv c, const uint64_t *pos, const uint64_t *d_np, uint64_t *out,
-                                               uint64_t *status)
+                                               uint64_t *status, ms_dev_meta *om)
 {
     const ms_parts pt = ms_parts_of(c.g, c.meta->count, c.meta->size_used, c.meta->size_compr);
     const uint64_t np = *d_np;
+    if (om && blockIdx.x == 0 && threadIdx.x == 0) {
+        om->count = np;
+        om->size_used = 8 * np;
+    }
     for (uint64_t i = (uint64_t)blockIdx.x * WG + threadIdx.x; i < np; i += (uint64_t)gridDim.x * WG) {
         const uint64_t p = pos[i];
         if (p >= pt.n) {
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(WG) void k_gather(ms_colv c, const uint64_t *pos, c
 }
 
 int launch_gather(const ms_col *data, const uint64_t *d_pos, const uint64_t *d_np, uint64_t np_bound,
-                  uint64_t *d_out, uint64_t *d_status, temps &sc)
+                  uint64_t *d_out, uint64_t *d_status, temps &sc, ms_dev_meta *om)
 {
     ms_colv v;
     MS_TRY(colv_of(data, v));
@@ -91,7 +95,7 @@ int launch_gather(const ms_col *data, const uint64_t *d_pos, const uint64_t *d_n
     if ((k == MS_DYNAMIC_VBP || k == MS_FOR) && !v.index)
         return ms_fail(MS_ERR_INVALID, "gather: column without a block index");
     hipLaunchKernelGGL(k_gather, dim3(grid_for(np_bound, WG * 4ull)), dim3(WG), 0, sc.s, v, d_pos, d_np, d_out,
-                       d_status);
+                       d_status, om);
     MS_HIP(hipGetLastError());
     return MS_OK;
 }

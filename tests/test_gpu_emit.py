@@ -57,3 +57,4 @@ def test_write_iterator_emission(oracle, f):
         g = ea.calc_binary(MS_OP_XOR, f, ea.upload_values(v), ea.upload_values(z))
         o = oracle.calc_binary(MS_OP_XOR, f, oracle.morph(ea.FormatDesc(0), v), oracle.morph(ea.FormatDesc(0), z))
         same(g, o)
+
