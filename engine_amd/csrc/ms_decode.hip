@@ -31,6 +31,46 @@ int launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t s)
     return MS_OK;
 }
 
+// The meta of a column of one uncompressed value (an aggregate's result).
+__device__ __forceinline__ void set_meta_one(ms_dev_meta *om, uint64_t compr)
+{
+    om->count = 1;
+    om->size_used = 8;
+    om->size_compr = compr;
+    om->status = 0;
+    for (int k = 0; k < 4; k++) om->aux[k] = 0;
+}
+
+// How a select + sum kernel ends.  Short columns run in one workgroup that
+// also takes the raw rest and writes the result, since the second launch
+// costs more than the sum (dynamic_vbp_f calls one after the other, two
+// launches / one: 1000 values 5.8 / 3.5 us, 8192 5.7 / 4.1, 16384 6.1 / 6.0;
+// delta_f at 16384 6.2 / 5.9).  Longer ones leave a partial sum per workgroup
+// to k_sum_finish (result null).
+struct ss_end {
+    uint64_t *part;
+    uint64_t *result;
+    ms_dev_meta *om;
+    uint64_t om_compr;
+    int with_rest;
+};
+constexpr uint64_t SS_SINGLE = 8192;
+
+__device__ __forceinline__ void ss_finish(const ms_colv &c, const ms_pred &p, const ss_end &end, uint64_t acc)
+{
+    if (!end.result) {
+        wg_partial(acc, end.part);
+        return;
+    }
+    if (end.with_rest) {
+        const ms_parts pt = parts_of(c);
+        const uint64_t *x = (const uint64_t *)(c.data + pt.rest_off);
+        for (uint64_t i = threadIdx.x; i < pt.n_rest; i += WG) acc += pred_eval(p, x[i]) ? x[i] : 0;
+    }
+    wg_partial(acc, end.result);   // one workgroup: its sum is the result
+    if (end.om && threadIdx.x == 0) set_meta_one(end.om, end.om_compr);
+}
+
 // One wave decodes one 512-value unit per iteration (grid-stride); the
 // next unit's index entry is fetched one iteration ahead.  Unit -> block
 // and block -> for_f block are shifts (the host only takes this path when
@@ -38,7 +78,7 @@ int launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t s)
 // predicate from a table built on the host; for_f specialises it per block
 // around the block's reference value.
 template <bool IS_FOR, bool LEFORM>
-__global__ __launch_bounds__(WG) void k_select_sum_blocks(ms_colv c, ms_pred p, ms_bwtab tab, uint64_t *res)
+__global__ __launch_bounds__(WG) void k_select_sum_blocks(ms_colv c, ms_pred p, ms_bwtab tab, ss_end end)
 {
     const ms_parts pt = parts_of(c);
     const uint32_t lg_spb = c.g.lg_spb;
@@ -75,12 +115,12 @@ __global__ __launch_bounds__(WG) void k_select_sum_blocks(ms_colv c, ms_pred p, 
         }
         vbp_units_ss<IS_FOR, LEFORM>(c.data, e, r, cnt, u0, mask, p, tab, j, gl, acc);
     }
-    wg_partial(acc, res);
+    ss_finish(c, p, end, acc);
 }
 
 // static_vbp_f<vbp_l<BW, S>> with 64 % S == 0.
 template <int BW>
-__global__ __launch_bounds__(WG) void k_select_sum_static(ms_colv c, ms_pred p, uint64_t *res)
+__global__ __launch_bounds__(WG) void k_select_sum_static(ms_colv c, ms_pred p, ss_end end)
 {
     const ms_parts pt = parts_of(c);
     const uint32_t S = c.g.lanes, lgS = c.g.lg_lanes;
@@ -117,11 +157,11 @@ __global__ __launch_bounds__(WG) void k_select_sum_static(ms_colv c, ms_pred p, 
             if (g < ngroups) ss_unit<BW>(base, S, j, g, cp, 0, acc);
         }
     }
-    wg_partial(acc, res);
+    ss_finish(c, p, end, acc);
 }
 
 // Uncompressed values: the whole of an uncompr_f column, or the rest part.
-__global__ __launch_bounds__(WG) void k_select_sum_uncompr(ms_colv c, ms_pred p, uint64_t *res)
+__global__ __launch_bounds__(WG) void k_select_sum_uncompr(ms_colv c, ms_pred p, ss_end end)
 {
     const ms_parts pt = parts_of(c);
     const uint64_t *x = (const uint64_t *)(c.data + pt.rest_off);
@@ -138,7 +178,7 @@ __global__ __launch_bounds__(WG) void k_select_sum_uncompr(ms_colv c, ms_pred p,
         const uint64_t v = x[2 * i];
         acc += pred_eval(p, v) ? v : 0;
     }
-    wg_partial(acc, res);
+    ss_finish(c, p, end, acc);
 }
 
 // *d_n decompressed values.
@@ -153,7 +193,7 @@ __global__ __launch_bounds__(WG) void k_select_sum_values(const uint64_t *x, con
 }
 
 // Any layout readable by read_compr, one value per thread.
-__global__ __launch_bounds__(WG) void k_select_sum_generic(ms_colv c, ms_pred p, uint64_t *res)
+__global__ __launch_bounds__(WG) void k_select_sum_generic(ms_colv c, ms_pred p, ss_end end)
 {
     const ms_parts pt = parts_of(c);
     uint64_t acc = 0;
@@ -161,13 +201,13 @@ __global__ __launch_bounds__(WG) void k_select_sum_generic(ms_colv c, ms_pred p,
         const uint64_t x = read_compr(c, i);
         if (pred_eval(p, x)) acc += x;
     }
-    wg_partial(acc, res);
+    ss_finish(c, p, end, acc);
 }
 
 // rle_f: a run of `len` copies of v contributes len * v when v passes.
 static constexpr uint64_t RLE_CHUNK = 512;   // runs per wave and step
 
-__global__ __launch_bounds__(WG) void k_select_sum_rle(ms_colv c, ms_pred p, uint64_t *res)
+__global__ __launch_bounds__(WG) void k_select_sum_rle(ms_colv c, ms_pred p, ss_end end)
 {
     const uint64_t runs = c.meta->size_used / 16;
     const u64x2 *w = (const u64x2 *)c.data;
@@ -179,7 +219,7 @@ __global__ __launch_bounds__(WG) void k_select_sum_rle(ms_colv c, ms_pred p, uin
         const uint64_t r0 = ch * RLE_CHUNK, r1 = r0 + RLE_CHUNK < runs ? r0 + RLE_CHUNK : runs;
         acc += rle_runs_ss(w, r0, r1, p, t);
     }
-    wg_partial(acc, res);
+    ss_finish(c, p, end, acc);
 }
 
 // ------------------------------------------------------------------
@@ -287,7 +327,7 @@ __global__ __launch_bounds__(WG) void k_delta_tiles(ms_colv c, const uint64_t *a
 
 // Select + sum over a delta_f column with 8 lanes and indexed 8-lane
 // inner blocks: one wave per tile, no workgroup synchronisation.
-__global__ __launch_bounds__(WG) void k_delta_select_sum(ms_colv c, ms_pred p, uint64_t *part)
+__global__ __launch_bounds__(WG) void k_delta_select_sum(ms_colv c, ms_pred p, ss_end end)
 {
     const ms_parts pt = parts_of(c);
     const uint64_t nunits = pt.n_compr >> 9;
@@ -305,7 +345,7 @@ __global__ __launch_bounds__(WG) void k_delta_select_sum(ms_colv c, ms_pred p, u
         delta_tile_ss<false>(c.data, my_e, c.refs, c.g.lg_spb, p, tile, nunits, t, j, gl, acc);
         my_e = e_next;
     }
-    wg_partial(acc, part);
+    ss_finish(c, p, end, acc);
 }
 
 // Per-tile lane totals, lane-major: sums[j * ntb + tile].
@@ -699,7 +739,7 @@ static bool fast_static(const ms_colv &v)
     return v.g.kind == MS_STATIC_VBP && v.g.lg_lanes != 0xff && v.g.lanes <= 64;
 }
 
-typedef void (*static_kernel_t)(ms_colv, ms_pred, uint64_t *);
+typedef void (*static_kernel_t)(ms_colv, ms_pred, ss_end);
 typedef void (*static_dec_t)(ms_colv, uint64_t *);
 
 static static_kernel_t static_sum_kernel(uint32_t bw)
@@ -724,15 +764,6 @@ static static_dec_t static_dec_kernel(uint32_t bw)
     }
 }
 
-// The meta of a column of one uncompressed value (an aggregate's result).
-__device__ __forceinline__ void set_meta_one(ms_dev_meta *om, uint64_t compr)
-{
-    om->count = 1;
-    om->size_used = 8;
-    om->size_compr = compr;
-    om->status = 0;
-    for (int k = 0; k < 4; k++) om->aux[k] = 0;
-}
 __global__ void k_set_meta_one(ms_dev_meta *om, uint64_t compr) { set_meta_one(om, compr); }
 
 // Sums the per-workgroup partials and the uncompressed rest (select + sum
@@ -855,26 +886,33 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
     const uint64_t nb = in->count_bound;
     uint32_t grid = 1;
     int with_rest = 1;
-    uint64_t *part = bufs ? bufs->part : (uint64_t *)sc.get(SS_MAX_PARTS * 8);
-    if (!part) return ms_fail(MS_ERR_NOMEM, "select_sum scratch");
+    // kinds whose kernels end with ss_finish (delta_f without a unit decoder
+    // and the formats read through decompression leave partial sums)
+    const bool ends = v.g.kind == MS_UNCOMPR || v.g.kind == MS_RLE || v.g.kind == MS_STATIC_VBP ||
+                      v.g.kind == MS_DYNAMIC_VBP || v.g.kind == MS_FOR || (v.g.kind == MS_DELTA && delta_fast(v));
+    const bool single = ends && nb <= SS_SINGLE;
+    uint64_t *part = single ? nullptr : bufs ? bufs->part : (uint64_t *)sc.get(SS_MAX_PARTS * 8);
+    if (!part && !single) return ms_fail(MS_ERR_NOMEM, "select_sum scratch");
+    const int rest = v.g.kind != MS_UNCOMPR && v.g.kind != MS_RLE;
+    const ss_end end = {part, single ? d_result : nullptr, om, om_compr, rest};
     switch (v.g.kind) {
     case MS_UNCOMPR:
         grid = grid_for(nb, WG * 32ull, 2048);
-        hipLaunchKernelGGL(k_select_sum_uncompr, dim3(grid), dim3(WG), 0, s, v, p, part);
+        hipLaunchKernelGGL(k_select_sum_uncompr, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
         with_rest = 0;
         break;
     case MS_RLE:
         grid = stride_grid((const void *)k_select_sum_rle, in->size_alloc / 16 / RLE_CHUNK + 1);
-        hipLaunchKernelGGL(k_select_sum_rle, dim3(grid), dim3(WG), 0, s, v, p, part);
+        hipLaunchKernelGGL(k_select_sum_rle, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
         with_rest = 0;
         break;
     case MS_STATIC_VBP:
         if (fast_static(v)) {
             grid = units_grid(nb);
-            hipLaunchKernelGGL(static_sum_kernel(v.g.bw), dim3(grid), dim3(WG), 0, s, v, p, part);
+            hipLaunchKernelGGL(static_sum_kernel(v.g.bw), dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
         } else {
             grid = grid_for(nb, WG * 16ull, 2048);
-            hipLaunchKernelGGL(k_select_sum_generic, dim3(grid), dim3(WG), 0, s, v, p, part);
+            hipLaunchKernelGGL(k_select_sum_generic, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
         }
         break;
     case MS_DYNAMIC_VBP:
@@ -886,10 +924,10 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
                    : v.g.kind == MS_FOR                    ? k_select_sum_blocks<true, false>
                                                            : k_select_sum_blocks<false, false>;
             grid = stride_grid((const void *)k, quads);
-            hipLaunchKernelGGL(k, dim3(grid), dim3(WG), 0, s, v, p, tab, part);
+            hipLaunchKernelGGL(k, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, tab, end);
         } else {
             grid = grid_for(nb, WG * 16ull, 2048);
-            hipLaunchKernelGGL(k_select_sum_generic, dim3(grid), dim3(WG), 0, s, v, p, part);
+            hipLaunchKernelGGL(k_select_sum_generic, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
         }
         break;
     case MS_DELTA: {
@@ -897,7 +935,7 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
         MS_TRY(delta_src(in, v, sc, &arr, bufs));
         if (!arr && v.g.lg_spb != 0xff) {
             grid = stride_grid((const void *)k_delta_select_sum, nb / DELTA_TILE + 1);
-            hipLaunchKernelGGL(k_delta_select_sum, dim3(grid), dim3(WG), 0, s, v, p, part);
+            hipLaunchKernelGGL(k_delta_select_sum, dim3(single ? 1 : grid), dim3(WG), 0, s, v, p, end);
             break;
         }
         grid = grid_for(nb / DELTA_TILE + 1, 2, 2048);
@@ -930,6 +968,7 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
         return ms_fail(MS_ERR_INVALID, "select_sum: unsupported format");
     }
     MS_HIP(hipGetLastError());
+    if (single) return MS_OK;
     static_assert(SS_MAX_PARTS >= 8192, "every grid above is capped at 8192 workgroups");
     hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(WG), 0, s, v, p, (const uint64_t *)part, grid, with_rest, d_result,
                        om, om_compr);
