@@ -1080,9 +1080,9 @@ int launch_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s, ms_dev_m
     return MS_OK;
 }
 
-// Flags of unit u's 512 values (bit t of the result's word m = value
-// 64 * (t >> 3) + 8 * m + (t & 7) of the unit, lane-major per thread):
-// decoded from the compressed part, or read raw from the rest.
+// Flags of unit u's 512 values, a byte per thread (bit m of thread t's byte
+// = value 64 * (t >> 3) + 8 * m + (t & 7) of the unit): decoded from the
+// compressed part, or read raw from the rest.
 // Index entry and for_f reference of unit u (left in vector registers, so
 // that a caller can request them one unit ahead and wait only at use).
 __device__ __forceinline__ void unit_entry(const ms_colv &c, uint64_t ncu, uint64_t u, uint64_t &e, uint64_t &r)
@@ -1097,69 +1097,212 @@ __device__ __forceinline__ void unit_entry(const ms_colv &c, uint64_t ncu, uint6
     }
 }
 
-__device__ __forceinline__ void unit_flags(const ms_colv &c, const ms_parts &pt, const ms_pred &p, uint64_t u,
-                                           uint64_t e_v, uint64_t r_v, uint32_t t, uint64_t (&B)[8])
+__device__ __forceinline__ uint32_t unit_flags(const ms_colv &c, const ms_parts &pt, const ms_pred &p, uint64_t u,
+                                               uint64_t e_v, uint64_t r_v, uint32_t t)
 {
     const uint32_t j = t & 7, gl = t >> 3;
     const uint64_t ncu = pt.n_compr >> 9;
     uint64_t d[8];
-    bool ok[8];
+    uint32_t ok = 0xff;
     if (u < ncu) {
         const uint64_t sub = u & ((1ull << c.g.lg_spb) - 1);
         const uint64_t e = uniform64(e_v);
         const uint64_t ref = c.g.kind == MS_FOR ? uniform64(r_v) : 0ull;
         dec_dispatch((uint32_t)(e & 0xff), (const uint64_t *)(c.data + (e >> 8)), 8, j, sub * 8 + gl, d);
 #pragma unroll
-        for (int m = 0; m < 8; m++) {
-            d[m] += ref;
-            ok[m] = true;
-        }
+        for (int m = 0; m < 8; m++) d[m] += ref;
     } else {
         // the raw rest: value i of the unit is rest value (u - ncu) * 512 + i
         const uint64_t *x = (const uint64_t *)(c.data + pt.rest_off);
         const uint64_t r0 = (u - ncu) * 512;
+        ok = 0;
 #pragma unroll
         for (int m = 0; m < 8; m++) {
             const uint64_t r = r0 + 64 * gl + 8 * m + j;
-            ok[m] = r < pt.n_rest;
-            d[m] = ok[m] ? gload(x + r) : 0ull;
+            const bool in = r < pt.n_rest;
+            d[m] = in ? gload(x + r) : 0ull;
+            ok |= in ? 1u << m : 0u;
         }
     }
+    uint32_t bits = 0;
 #pragma unroll
-    for (int m = 0; m < 8; m++) B[m] = __ballot(ok[m] && pred_eval(p, d[m]));
+    for (int m = 7; m >= 0; m--) bits = bits + bits + (pred_eval(p, d[m]) ? 1u : 0u);
+    return bits & ok;
 }
 
+// The flags of a thread's 8 codes (at most 32 bits, cut from its words), bit
+// m for code m, under the unit's predicate mode.
+template <int BW>
+__device__ __forceinline__ uint32_t flag_cut(const uint64_t (&w)[5], uint32_t g, uint32_t mode, uint32_t lo,
+                                             uint32_t span)
+{
+    uint32_t c[8], bits = 0;
+    vbp_cut32<BW>(w, ((g * BW) & 7) * 8, c);
+    if (mode == SM_LE) {
+#pragma unroll
+        for (int m = 7; m >= 0; m--) bits = bits + bits + (c[m] <= span ? 1u : 0u);
+    } else {
+#pragma unroll
+        for (int m = 7; m >= 0; m--) bits = bits + bits + ((uint32_t)(c[m] - lo) <= span ? 1u : 0u);
+    }
+    return bits;
+}
 
-// Decodes and tests every unit once: its 8 ballots go to flags[8 u ..]
-// (64 bytes per 512 values) and its selected count to cnt[u].
-__global__ __launch_bounds__(WG) void k_sel_count_blocks(ms_colv c, ms_pred p, uint64_t *d_units, uint64_t *cnt,
-                                                         uint64_t *flags)
+__device__ __forceinline__ uint32_t flag_cut_dispatch(uint32_t bw, const uint64_t (&w)[5], uint32_t g, uint32_t mode,
+                                                      uint32_t lo, uint32_t span)
+{
+    switch (bw) {
+#define MS_CASE(X) \
+    case X: return flag_cut<X>(w, g, mode, lo, span);
+        MS_BW32_CASES(MS_CASE)
+#undef MS_CASE
+    default: return 0;
+    }
+}
+
+// A unit's predicate mode and its words' request for k_sel_count_blocks: the
+// fused sums' own, but that a wholly selected unit is not read either.
+template <bool IS_FOR>
+__device__ __forceinline__ void flag_prep(const uint8_t *data, uint64_t e, uint64_t r, bool valid, uint64_t u,
+                                          uint64_t mask, const ms_pred &p, const ms_bwtab &tab, uint32_t j,
+                                          uint32_t gl, uint32_t &mode, uint32_t &lo, uint32_t &span,
+                                          uint64_t (&w)[5])
+{
+    mode = SM_NONE;
+    lo = span = 0;
+    if (!valid) return;
+    const uint32_t bw = (uint32_t)(e & 0xff);
+    if (bw > 32) {
+        mode = SM_SLOW;
+    } else if (IS_FOR) {
+        const uint64_t maxcode = (1ull << bw) - 1ull;
+        if (r + maxcode < r) {
+            mode = SM_SLOW;
+        } else {
+            const ms_cpred cp = code_pred(p, r, maxcode);
+            mode = cp.mode == PM_NONE ? SM_NONE : cp.mode == PM_ALL ? SM_ALL : cp.mode == PM_OUT ? SM_OUT
+                 : cp.clo == 0 ? SM_LE : SM_IN;
+            lo = (uint32_t)cp.clo;
+            span = (uint32_t)cp.cspan;
+        }
+    } else {
+        mode = tab.mode[bw];
+        lo = tab.lo[bw];
+        span = tab.span[bw];
+    }
+    if (mode == SM_LE || mode == SM_IN || mode == SM_OUT) {
+        uint32_t g = (uint32_t)(u & mask) * 8 + gl;
+        asm volatile("" : "+v"(g));   // keeps per-width offsets of g from being hoisted
+        unit_words_dispatch(bw, (const uint64_t *)(data + (e >> 8)), j, g, w);
+    }
+}
+
+// The flags of a thread's 8 wide (more than 32 bits) or wrapping codes.  Out
+// of line, as the fused sums' rare path is, so that it does not set the
+// kernel's register budget.
+__device__ __attribute__((noinline, pure)) uint32_t slow_flags(const ms_pred p, const uint64_t *base, uint32_t bw, uint32_t j,
+                                                         uint32_t g, uint64_t ref)
+{
+    uint64_t d[8];
+    dec_dispatch(bw, base, 8, j, g, d);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int m = 7; m >= 0; m--) bits = bits + bits + (pred_eval(p, d[m] + ref) ? 1u : 0u);
+    return bits;
+}
+
+// The flags of a thread's 8 codes of unit u.
+template <bool IS_FOR>
+__device__ __forceinline__ uint32_t flag_finish(const uint8_t *data, const ms_pred &p, uint64_t e, uint64_t r,
+                                                bool valid, uint64_t u, uint64_t mask, uint32_t j, uint32_t gl,
+                                                uint32_t mode, uint32_t lo, uint32_t span, const uint64_t (&w)[5])
+{
+    if (!valid || mode == SM_NONE) return 0;
+    if (mode == SM_ALL) return 0xff;
+    uint32_t g = (uint32_t)(u & mask) * 8 + gl;
+    asm volatile("" : "+v"(g));
+    const uint32_t bw = (uint32_t)(e & 0xff);
+    if (mode == SM_SLOW) return slow_flags(p, (const uint64_t *)(data + (e >> 8)), bw, j, g, IS_FOR ? r : 0ull);
+    const uint32_t bits = flag_cut_dispatch(bw, w, g, mode, lo, span);
+    return mode == SM_OUT ? bits ^ 0xffu : bits;
+}
+
+// Sum over the wave (DPP), uniform.
+__device__ __forceinline__ uint32_t dpp_sum_u32(uint32_t x)
+{
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Decodes and tests every unit once: each thread's flag byte goes to byte t
+// of the unit's flags (64 bytes per 512 values) and its selected count to
+// cnt[u].  As the fused sums do, a wave takes 4 units at a time: each unit's
+// predicate is reduced to its codes' range, the words of all 4 are requested
+// before the first is cut (none for a unit that is selected wholly or not at
+// all), and codes of up to 32 bits are tested in 32 bits.
+// Bound by the decode's instructions (3-bit codes) or HBM (20 bits: 4.1
+// TB/s).  Measured for 2^28 rows, one unit at a time in 64 bits with a ballot
+// word per code before / now: 3-bit codes 164 / 102 us, 20-bit codes 226 /
+// 163 us; for_f of 2^26 rows 47 / 38 us.
+template <bool IS_FOR>
+__global__ __launch_bounds__(WG) void k_sel_count_blocks(ms_colv c, ms_pred p, ms_bwtab tab, uint64_t *d_units,
+                                                         uint64_t *cnt, uint64_t *flags)
 {
     const ms_parts pt = parts_of(c);
     const uint64_t nunits = (pt.n + 511) / 512;
     const uint64_t ncu = pt.n_compr >> 9;
+    const uint64_t nq = (ncu + 3) >> 2;   // groups of 4 packed units
     const uint32_t t = threadIdx.x & 63;
+    const uint32_t j = t & 7, gl = t >> 3;
     const uint64_t W = (uint64_t)gridDim.x * WAVES;
-    uint64_t u = (uint64_t)blockIdx.x * WAVES + wave_index();
+    const uint64_t first = (uint64_t)blockIdx.x * WAVES + wave_index();
+    const uint64_t mask = (1ull << c.g.lg_spb) - 1ull;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *d_units = nunits;   // for the scan and the compaction after this kernel
+        *d_units = nunits;   // for the scan and the emission after this kernel
         cnt[nunits] = 0;     // the scan's total slot
     }
-    uint64_t e_n, r_n;   // the next unit's entry, requested one unit ahead
-    unit_entry(c, ncu, u, e_n, r_n);
-    for (; u < nunits; u += W) {
-        const uint64_t e_v = e_n, r_v = r_n;
-        unit_entry(c, ncu, u + W, e_n, r_n);
-        uint64_t B[8];
-        unit_flags(c, pt, p, u, e_v, r_v, t, B);
-        uint32_t n = 0;
-        uint64_t mine = 0;
+    uint64_t my_e = 0, my_r = 0;   // lanes 0..3: the next group's entries, requested one group ahead
+    if (first < nq && t < 4) unit_entry(c, ncu, first * 4 + t, my_e, my_r);
+    for (uint64_t q = first; q < nq; q += W) {
+        const uint64_t u0 = q * 4;
+        const uint32_t num = ncu - u0 < 4 ? (uint32_t)(ncu - u0) : 4u;
+        uint64_t e[4], r[4];
 #pragma unroll
-        for (int m = 0; m < 8; m++) {
-            n += __popcll(B[m]);
-            if (t == (uint32_t)m) mine = B[m];
+        for (int k = 0; k < 4; k++) {
+            e[k] = readlane64(my_e, k);
+            r[k] = IS_FOR ? readlane64(my_r, k) : 0ull;
         }
-        if (t < 8) flags[8 * u + t] = mine;
+        my_e = my_r = 0;
+        if (q + W < nq && t < 4) unit_entry(c, ncu, u0 + 4 * W + t, my_e, my_r);
+        uint32_t mo0, mo1, mo2, mo3, lo0, lo1, lo2, lo3, sp0, sp1, sp2, sp3;
+        uint64_t w0[5], w1[5], w2[5], w3[5];   // named arrays: they stay in registers
+        flag_prep<IS_FOR>(c.data, e[0], r[0], num > 0, u0, mask, p, tab, j, gl, mo0, lo0, sp0, w0);
+        flag_prep<IS_FOR>(c.data, e[1], r[1], num > 1, u0 + 1, mask, p, tab, j, gl, mo1, lo1, sp1, w1);
+        flag_prep<IS_FOR>(c.data, e[2], r[2], num > 2, u0 + 2, mask, p, tab, j, gl, mo2, lo2, sp2, w2);
+        flag_prep<IS_FOR>(c.data, e[3], r[3], num > 3, u0 + 3, mask, p, tab, j, gl, mo3, lo3, sp3, w3);
+        const uint32_t f0 = flag_finish<IS_FOR>(c.data, p, e[0], r[0], num > 0, u0, mask, j, gl, mo0, lo0, sp0, w0);
+        const uint32_t f1 = flag_finish<IS_FOR>(c.data, p, e[1], r[1], num > 1, u0 + 1, mask, j, gl, mo1, lo1, sp1, w1);
+        const uint32_t f2 = flag_finish<IS_FOR>(c.data, p, e[2], r[2], num > 2, u0 + 2, mask, j, gl, mo2, lo2, sp2, w2);
+        const uint32_t f3 = flag_finish<IS_FOR>(c.data, p, e[3], r[3], num > 3, u0 + 3, mask, j, gl, mo3, lo3, sp3, w3);
+        uint8_t *fb = (uint8_t *)(flags + 8 * u0) + t;
+        fb[0] = (uint8_t)f0;
+        if (num > 1) fb[64] = (uint8_t)f1;
+        if (num > 2) fb[128] = (uint8_t)f2;
+        if (num > 3) fb[192] = (uint8_t)f3;
+        const uint32_t n01 = dpp_sum_u32((uint32_t)__builtin_popcount(f0) + ((uint32_t)__builtin_popcount(f1) << 16));
+        const uint32_t n23 = dpp_sum_u32((uint32_t)__builtin_popcount(f2) + ((uint32_t)__builtin_popcount(f3) << 16));
+        const uint32_t pair = t & 2 ? n23 : n01;
+        if (t < num) cnt[u0 + t] = t & 1 ? pair >> 16 : pair & 0xffffu;
+    }
+    for (uint64_t u = ncu + first; u < nunits; u += W) {   // the raw rest
+        const uint32_t f = unit_flags(c, pt, p, u, 0, 0, t);
+        ((uint8_t *)(flags + 8 * u))[t] = (uint8_t)f;
+        const uint32_t n = dpp_sum_u32((uint32_t)__builtin_popcount(f));
         if (t == 0) cnt[u] = n;
     }
 }
@@ -1222,16 +1365,9 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void k_select_onepass(ms_colv c, co
                     continue;
                 }
                 if (SRC == SEL_LANES8) {
-                    uint64_t B[8];
-                    unit_flags(c, pt, p, u, readlane64(my_e, k), readlane64(my_r, k), t, B);
-                    // byte gl of ballot m holds rows 64 gl + 8 m ..: byte m of row word gl
-                    uint64_t mine = B[0];
-#pragma unroll
-                    for (uint32_t m = 0; m < 8; m++) {
-                        n += (uint32_t)__popcll(B[m]);
-                        if (m && (t >> 3) == m) mine = B[m];
-                    }
-                    ((uint8_t *)rows)[8 * (t & 7) + (t >> 3)] = (uint8_t)(mine >> (8 * (t & 7)));
+                    const uint32_t f = unit_flags(c, pt, p, u, readlane64(my_e, k), readlane64(my_r, k), t);
+                    ((uint8_t *)rows)[t] = (uint8_t)f;
+                    n += dpp_sum_u32((uint32_t)__builtin_popcount(f));
                 } else if (SRC == SEL_LANES1) {
                     // thread t holds rows 8 t .. 8 t + 7: wholly packed or wholly raw
                     // (the packed part is a multiple of 64)
@@ -1301,7 +1437,8 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void k_select_onepass(ms_colv c, co
             uint64_t o = readlane64(s_base, 0) + pmine;
             const uint64_t u0 = ptile * tile_units + w * per_wave;
             // the wave's row words, one per lane
-            const uint64_t mine_w = (&s_rows[turn ^ 1][w][0][0])[t % (8 * SEL_UNITS)];
+            uint64_t mine_w = (&s_rows[turn ^ 1][w][0][0])[t % (8 * SEL_UNITS)];
+            if (SRC == SEL_LANES8) mine_w = flag_rows(mine_w);
 #pragma unroll 4
             for (uint32_t r = 0; r < 8 * per_wave; r++) {
                 const uint64_t F = readlane64(mine_w, r);
@@ -1355,7 +1492,9 @@ int launch_select_flags(const ms_col *in, const ms_pred &p, sel_flags &sf, temps
     uint64_t *off = (uint64_t *)sc.get(units * 8 + 64);
     uint64_t *flags = (uint64_t *)sc.get(units * 64 + 64);
     if (!d_u || !cnt || !off || !flags) return ms_fail(MS_ERR_NOMEM, "select scratch");
-    hipLaunchKernelGGL(k_sel_count_blocks, dim3(units_grid(nb)), dim3(WG), 0, s, v, p, d_u, cnt, flags);
+    auto k = v.g.kind == MS_FOR ? k_sel_count_blocks<true> : k_sel_count_blocks<false>;
+    hipLaunchKernelGGL(k, dim3(stride_grid((const void *)k, nb / 2048 + 1)), dim3(WG), 0, s, v, p, make_bwtab(p), d_u,
+                       cnt, flags);
     MS_HIP(hipGetLastError());
     MS_TRY(launch_exclusive_scan_n(cnt, off, d_u, 1, units + 1, sc));
     sf.flags = flags;

@@ -180,6 +180,18 @@ __device__ __forceinline__ uint64_t wave_or_u64(uint64_t x)
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
+// Bit m of byte j to bit j of byte m (an 8 x 8 transpose in three swaps of
+// ever larger blocks): a select's flag word to its 64 rows in order.
+__device__ __forceinline__ uint64_t flag_rows(uint64_t x)
+{
+    uint64_t y = (x ^ (x >> 7)) & 0x00aa00aa00aa00aaull;
+    x ^= y ^ (y << 7);
+    y = (x ^ (x >> 14)) & 0x0000cccc0000ccccull;
+    x ^= y ^ (y << 14);
+    y = (x ^ (x >> 28)) & 0x00000000f0f0f0f0ull;
+    return x ^ y ^ (y << 28);
+}
+
 // Predicate of select as a value range [lo, hi], optionally negated:
 // EQ [v,v]; NE !(EQ); LT [0,v-1]; LE [0,v]; GT [v+1,MAX]; GE [v,MAX].
 struct ms_pred {

@@ -159,11 +159,10 @@ __device__ __forceinline__ uint64_t flag_r0(const emit_layout &l, const flag_src
 // One wave writes the rows of ranks [r0, r0 + cnt) to st(rank - r0, row),
 // walking the units from u (a unit at or before the one holding rank r0)
 // eight at a time.  Lane t takes rows 64 gl .. 64 gl + 63 of unit
-// u + t / 8 (gl = t & 7): row 64 gl + 8 m + j of a unit is bit 8 gl + j of
-// its ballot m (the count pass's thread mapping), so the lane's row word
-// is byte gl of each of the unit's 8 ballots.  Its first rank is the
-// unit's offset plus the set bits of the unit's lower row words (a scan
-// over the lane's group of 8); then it writes its set bits in order.
+// u + t / 8 (gl = t & 7): its flag word, whose bits flag_rows puts in row
+// order.  Its first rank is the unit's offset plus the set bits of the
+// unit's lower row words (a scan over the lane's group of 8); then it
+// writes its set bits in order.
 template <class St>
 __device__ __forceinline__ void gather_ranks(const sel_flags &sf, uint64_t nunits, uint64_t u, uint64_t r0,
                                              uint64_t cnt, const St &st)
@@ -177,13 +176,8 @@ __device__ __forceinline__ void gather_ranks(const sel_flags &sf, uint64_t nunit
         const uint64_t end_rank = gload(sf.uoff + ue);   // requested with the group's loads
         uint64_t rw = 0, rank = 0;
         if (uu < nunits) {
-            uint64_t b[8];
-#pragma unroll
-            for (int m = 0; m < 8; m++) b[m] = gload(sf.flags + 8 * uu + m);
+            rw = flag_rows(gload(sf.flags + 8 * uu + gl));
             rank = gload(sf.uoff + uu);
-            const uint32_t sh = 8 * gl;
-#pragma unroll
-            for (int m = 0; m < 8; m++) rw |= ((b[m] >> sh) & 0xffull) << (8 * m);
         }
         // exclusive scan of the row words' counts within the group of 8
         const uint32_t c = (uint32_t)__popcll(rw);
@@ -219,7 +213,7 @@ __device__ __forceinline__ void gather_ranks(const sel_flags &sf, uint64_t nunit
 
 // The select's split (thread 0): the selected rows below the scalar
 // remainder's first row thr are counted from the unit offsets and thr's
-// unit's ballots.
+// unit's flags.
 __device__ __forceinline__ void select_split(const sel_flags &sf, const sel_split &sp, uint64_t nunits)
 {
     const ms_dev_meta *in = sp.in_meta;
@@ -232,15 +226,9 @@ __device__ __forceinline__ void select_split(const sel_flags &sf, const sel_spli
     const uint64_t u = thr / 512, w = thr % 512;
     uint64_t na = u < nunits ? sf.uoff[u] : total;
     if (u < nunits && w) {
-        // row 64 gl + 8 m + j of the unit is bit 8 gl + j of ballot m
-        for (uint32_t m = 0; m < 8; m++) {
-            const uint64_t B = sf.flags[8 * u + m];
-            for (uint32_t gl = 0; gl < 8; gl++) {
-                const uint64_t row = 64 * gl + 8 * m;
-                if (row >= w) continue;
-                const uint64_t k = w - row < 8 ? w - row : 8;
-                na += __popcll((B >> (8 * gl)) & ((1ull << k) - 1));
-            }
+        for (uint32_t gl = 0; 64 * gl < w; gl++) {
+            const uint64_t k = w - 64 * gl;   // rows of the word below thr
+            na += __popcll(flag_rows(sf.flags[8 * u + gl]) & (k < 64 ? (1ull << k) - 1 : ~0ull));
         }
     }
     *sp.d_cnt = total;

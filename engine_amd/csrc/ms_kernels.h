@@ -71,8 +71,9 @@ int launch_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s, ms_dev_m
 int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos, uint64_t *d_cnt, temps &sc,
                             ms_dev_meta *om = nullptr);
 // The selected rows of a select as its count pass leaves them, without
-// materialising positions: 8 ballots per 512-row unit (bit 8 gl + j of
-// ballot m = row 64 gl + 8 m + j of the unit) and uoff[u] = the number of
+// materialising positions: 8 words per 512-row unit (bit m of byte j of word
+// gl = row 64 gl + 8 m + j of the unit: the count pass's threads write a byte
+// each; flag_rows gives word gl's rows in order) and uoff[u] = the number of
 // selected rows before unit u (uoff[*d_units] = all of them).  Ranks are
 // positions in the select's ascending output.
 struct sel_flags {
