@@ -14,6 +14,7 @@
 //   calc       : element-wise op mod 2^64 (scalar/calc_uncompr.h:98-100).
 #include "ms_kernels.h"
 #include "ms_lookback.hpp"
+#include "ms_merge_path.hpp"
 
 namespace ms {
 
@@ -287,31 +288,23 @@ int launch_intersect(const uint64_t *a, const uint64_t *d_na, uint64_t na_bound,
 // values a thread.  Every value of a is kept; b's value of rank r among its
 // equals is kept unless a holds more than r of them, which in merged order is
 // whether a's value r + 1 places back equals it.  A look-back over the tiles'
-// kept values places the output.
+// kept values places the output.  Lists that are not ascending have no
+// union, but every access stays inside them (merge_part_of).
 // Bound by the merge in LDS and the tiles' chain of steps; one search per
 // value in global memory (rank flags, a scan, places) took 620 us for 2.9
 // and 8.4 10^6 positions, this takes 83 us (4096 values a tile: 106 us).
 constexpr uint32_t MRG_WG = 1024, MRG_PER = 8, MRG_TILE = MRG_WG * MRG_PER;
 
-// Values of a among the first d of the merged order (one wave, uniform).
-__device__ __forceinline__ uint64_t merge_split(const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb,
-                                                uint64_t d)
-{
-    const uint32_t t = lane_id();
-    uint64_t lo = d > nb ? d - nb : 0, hi = d < na ? d : na;
-    while (lo < hi) {
-        const uint64_t span = hi - lo;
-        const bool fine = span <= 64;
-        const uint64_t i = fine ? lo + t : lo + span * t / 64;
-        const bool in = i < hi && gload(a + i) <= gload(b + (d - 1 - i));   // true up to the split
-        const uint32_t c = (uint32_t)__popcll(__ballot(in));
-        if (fine) return lo + c;
-        const uint64_t nlo = c ? lo + span * (c - 1) / 64 + 1 : lo, nhi = c < 64 ? lo + span * c / 64 : hi;
-        lo = nlo;
-        hi = nhi;
+// merge_split's count over lists in global memory (one wave, uniform).
+struct merge_count {
+    const uint64_t *a, *b;
+    __device__ __forceinline__ uint32_t operator()(uint64_t lo, uint64_t span, uint64_t d) const
+    {
+        const uint64_t i = merge_probe(lo, span, lane_id());
+        const bool in = i < lo + span && gload(a + i) <= gload(b + (d - 1 - i));
+        return (uint32_t)__popcll(__ballot(in));
     }
-    return lo;
-}
+};
 
 __global__ __launch_bounds__(MRG_WG, 8) void k_merge(const uint64_t *a, const uint64_t *d_na, const uint64_t *b,
                                                   const uint64_t *d_nb, uint64_t *state, uint64_t *out,
@@ -331,12 +324,13 @@ __global__ __launch_bounds__(MRG_WG, 8) void k_merge(const uint64_t *a, const ui
         if (tile >= ntiles) return;
         const uint64_t d0 = tile * MRG_TILE, d1 = d0 + MRG_TILE < n ? d0 + MRG_TILE : n;
         if (w < 2) {
-            const uint64_t sp = merge_split(a, na, b, nb, w ? d1 : d0);
+            const uint64_t sp = merge_split(na, nb, w ? d1 : d0, merge_count{a, b});
             if (t == 0) s_split[w] = sp;
         }
         __syncthreads();
-        const uint64_t a0 = readlane64(s_split[0], 0), b0 = d0 - a0;
-        const uint32_t la = (uint32_t)(readlane64(s_split[1], 0) - a0), len = (uint32_t)(d1 - d0), lb = len - la;
+        const merge_part pt = merge_part_of(readlane64(s_split[0], 0), readlane64(s_split[1], 0), d0, d1, na, nb);
+        const uint64_t a0 = pt.a0, b0 = pt.b0;
+        const uint32_t la = pt.la, lb = pt.lb, len = la + lb;   // all of d1 - d0 with ascending lists
 #pragma unroll
         for (uint32_t q = 0; q < MRG_PER; q++) {
             const uint32_t i = q * MRG_WG + threadIdx.x;
