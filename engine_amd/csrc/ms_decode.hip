@@ -55,6 +55,12 @@ struct ss_end {
     int with_rest;
 };
 constexpr uint64_t SS_SINGLE = 8192;
+// Layouts read value by value (k_select_sum_generic) are bound by the reads
+// themselves: beyond what one workgroup of their two launches takes, a second
+// one is worth more than the launch (two launches / one: dynamic_vbp_f<64, 8,
+// 1> 4096 values 12.4 / 10.2 us, 4608 9.2 / 11.2, 8192 12.6 / 18.3; for_f over
+// uncompr_f 4096 14.9 / 12.4, 4608 10.8 / 13.7, 8192 15.2 / 22.8).
+constexpr uint64_t SS_SINGLE_GENERIC = WG * 16;
 
 __device__ __forceinline__ void ss_finish(const ms_colv &c, const ms_pred &p, const ss_end &end, uint64_t acc)
 {
@@ -890,7 +896,9 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
     // and the formats read through decompression leave partial sums)
     const bool ends = v.g.kind == MS_UNCOMPR || v.g.kind == MS_RLE || v.g.kind == MS_STATIC_VBP ||
                       v.g.kind == MS_DYNAMIC_VBP || v.g.kind == MS_FOR || (v.g.kind == MS_DELTA && delta_fast(v));
-    const bool single = ends && nb <= SS_SINGLE;
+    const bool by_value = v.g.kind == MS_STATIC_VBP ? !fast_static(v)
+                        : (v.g.kind == MS_DYNAMIC_VBP || v.g.kind == MS_FOR) && !fast_blocks(v);
+    const bool single = ends && nb <= (by_value ? SS_SINGLE_GENERIC : SS_SINGLE);
     uint64_t *part = single ? nullptr : bufs ? bufs->part : (uint64_t *)sc.get(SS_MAX_PARTS * 8);
     if (!part && !single) return ms_fail(MS_ERR_NOMEM, "select_sum scratch");
     const int rest = v.g.kind != MS_UNCOMPR && v.g.kind != MS_RLE;
