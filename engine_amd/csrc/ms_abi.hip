@@ -474,18 +474,18 @@ static int new_col(const ms_format_desc &f, uint64_t count_bound, uint64_t size_
     const uint64_t refs_bytes = (c->refs_cap * 8 + 255) / 256 * 256;
     const uint64_t tab_bytes = caps ? (caps->tab_bytes + 255) / 256 * 256 : 0;
     const uint64_t data_bytes = (size_alloc + 1024 + 255) / 256 * 256;
-    uint8_t *base = (uint8_t *)dev_alloc(256 + idx_bytes + refs_bytes + tab_bytes + data_bytes, s);
+    uint8_t *base = (uint8_t *)dev_alloc(COL_META_BYTES + idx_bytes + refs_bytes + tab_bytes + data_bytes, s);
     if (!base) {
         delete c;
         return ms_fail(MS_ERR_NOMEM, "device allocation of %llu bytes", (unsigned long long)(size_alloc + 1024));
     }
     c->arena = g_rec && g_rec->recording && g_rec->mode == 1 ? g_rec : nullptr;
     c->meta = (ms_dev_meta *)base;
-    c->index = c->index_cap ? (uint64_t *)(base + 256) : nullptr;
-    c->refs = c->refs_cap ? (uint64_t *)(base + 256 + idx_bytes) : nullptr;
-    c->vmeta = tab_bytes ? (ms_dev_meta *)(base + 256 + idx_bytes + refs_bytes) : nullptr;
-    c->data = base + 256 + idx_bytes + refs_bytes + tab_bytes;
-    int rc = clear_meta ? launch_fill_u64((uint64_t *)base, 256 / 8, 0, s) : MS_OK;
+    c->index = c->index_cap ? (uint64_t *)(base + COL_META_BYTES) : nullptr;
+    c->refs = c->refs_cap ? (uint64_t *)(base + COL_META_BYTES + idx_bytes) : nullptr;
+    c->vmeta = tab_bytes ? (ms_dev_meta *)(base + COL_META_BYTES + idx_bytes + refs_bytes) : nullptr;
+    c->data = base + COL_META_BYTES + idx_bytes + refs_bytes + tab_bytes;
+    int rc = clear_meta ? launch_fill_u64((uint64_t *)base, COL_META_BYTES / 8, 0, s) : MS_OK;
     if (rc) {
         dev_free(base, s);
         delete c;
@@ -1506,9 +1506,7 @@ extern "C" int ms_agg_sum(ms_col **out, const ms_col *in, void *stream)
     ms_col *c;
     MS_TRY(new_col(uncompr_desc(), 1, 64, S(stream), &c, nullptr, false));
     ms_pred all = make_pred(MS_CMP_GE, 0);
-    // agg_sum_compr.h:148-150 vs agg_sum_uncompr.h:126 (sizeCompr 8 vs 0)
-    const int rc = launch_select_sum(in, all, (uint64_t *)c->data, false, S(stream), nullptr, c->meta,
-                                     in->f.kind == MS_UNCOMPR ? 0ull : 8ull);
+    const int rc = launch_select_sum(in, all, (uint64_t *)c->data, false, S(stream), nullptr, true);
     if (rc) { ms_col_free(c); return rc; }
     *out = c;
     return MS_OK;

@@ -31,12 +31,15 @@ int launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t s)
     return MS_OK;
 }
 
-// The meta of a column of one uncompressed value (an aggregate's result).
-__device__ __forceinline__ void set_meta_one(ms_dev_meta *om, uint64_t compr)
+// The meta of the uncompr_f column whose one value is at `value`, the sum of
+// a column of format kind `of` (sizeCompr: agg_sum_compr.h:148-150 vs
+// agg_sum_uncompr.h:126).
+__device__ __forceinline__ void set_meta_one(uint64_t *value, uint32_t of)
 {
+    ms_dev_meta *om = (ms_dev_meta *)((uint8_t *)value - COL_META_BYTES);
     om->count = 1;
     om->size_used = 8;
-    om->size_compr = compr;
+    om->size_compr = of == MS_UNCOMPR ? 0 : 8;
     om->status = 0;
     for (int k = 0; k < 4; k++) om->aux[k] = 0;
 }
@@ -46,14 +49,14 @@ __device__ __forceinline__ void set_meta_one(ms_dev_meta *om, uint64_t compr)
 // costs more than the sum (dynamic_vbp_f calls one after the other, two
 // launches / one: 1000 values 5.8 / 3.5 us, 8192 5.7 / 4.1, 16384 6.1 / 6.0;
 // delta_f at 16384 6.2 / 5.9).  Longer ones leave a partial sum per workgroup
-// to k_sum_finish (result null).
-struct ss_end {
-    uint64_t *part;
-    uint64_t *result;
-    ms_dev_meta *om;
-    uint64_t om_compr;
-    int with_rest;
-};
+// to k_sum_finish.  One word says which, so that the launches of longer sums
+// carry no more arguments than their own: the address of the partial sums or
+// of the result, SS_RESULT for the latter and SS_META if that is the value of
+// a column (addresses have 57 bits at most).  48 bytes of arguments more in
+// the two launches cost 0.6 to 0.9 us of 8 where the host is the slower side
+// (100,000 values of static_vbp_f<20, 8>: 8.5 -> 9.1 us, now 8.4).
+typedef uint64_t ss_end;
+constexpr uint64_t SS_RESULT = 1ull << 63, SS_META = 1ull << 62;
 constexpr uint64_t SS_SINGLE = 8192;
 // Layouts read value by value (k_select_sum_generic) are bound by the reads
 // themselves: beyond what one workgroup of their two launches takes, a second
@@ -62,19 +65,16 @@ constexpr uint64_t SS_SINGLE = 8192;
 // uncompr_f 4096 14.9 / 12.4, 4608 10.8 / 13.7, 8192 15.2 / 22.8).
 constexpr uint64_t SS_SINGLE_GENERIC = WG * 16;
 
-__device__ __forceinline__ void ss_finish(const ms_colv &c, const ms_pred &p, const ss_end &end, uint64_t acc)
+__device__ __forceinline__ void ss_finish(const ms_colv &c, const ms_pred &p, ss_end end, uint64_t acc)
 {
-    if (!end.result) {
-        wg_partial(acc, end.part);
-        return;
-    }
-    if (end.with_rest) {
+    uint64_t *dst = (uint64_t *)(end & ~(SS_RESULT | SS_META));
+    if ((end & SS_RESULT) && c.g.kind != MS_UNCOMPR && c.g.kind != MS_RLE) {
         const ms_parts pt = parts_of(c);
         const uint64_t *x = (const uint64_t *)(c.data + pt.rest_off);
         for (uint64_t i = threadIdx.x; i < pt.n_rest; i += WG) acc += pred_eval(p, x[i]) ? x[i] : 0;
     }
-    wg_partial(acc, end.result);   // one workgroup: its sum is the result
-    if (end.om && threadIdx.x == 0) set_meta_one(end.om, end.om_compr);
+    wg_partial(acc, dst);   // one workgroup: its sum is the result
+    if ((end & SS_META) && threadIdx.x == 0) set_meta_one(dst, c.g.kind);
 }
 
 // One wave decodes one 512-value unit per iteration (grid-stride); the
@@ -770,13 +770,13 @@ static static_dec_t static_dec_kernel(uint32_t bw)
     }
 }
 
-__global__ void k_set_meta_one(ms_dev_meta *om, uint64_t compr) { set_meta_one(om, compr); }
+__global__ void k_set_meta_one(uint64_t *value, uint32_t of) { set_meta_one(value, of); }
 
 // Sums the per-workgroup partials and the uncompressed rest (select + sum
 // over the rest part, the vectorised and scalar loops of
 // agg_sum_compr.h:110-146 folded into one) and writes the result.
 __global__ __launch_bounds__(WG) void k_sum_finish(ms_colv c, ms_pred p, const uint64_t *part, uint32_t nparts,
-                                                   int with_rest, uint64_t *result, ms_dev_meta *om, uint64_t om_compr)
+                                                   int with_rest, ss_end end)
 {
     uint64_t acc = 0;
     for (uint32_t i = threadIdx.x; i < nparts; i += WG) acc += part[i];
@@ -792,8 +792,9 @@ __global__ __launch_bounds__(WG) void k_sum_finish(ms_colv c, ms_pred p, const u
     if (threadIdx.x == 0) {
         uint64_t sum = 0;
         for (int w = 0; w < WAVES; w++) sum += s_part[w];
+        uint64_t *result = (uint64_t *)(end & ~SS_META);
         *result = sum;
-        if (om) set_meta_one(om, om_compr);
+        if (end & SS_META) set_meta_one(result, c.g.kind);
     }
 }
 
@@ -877,14 +878,14 @@ static uint32_t stride_grid(const void *kernel, uint64_t items)
 }
 
 int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bool accumulate, hipStream_t s,
-                      const ss_buffers *bufs, ms_dev_meta *om, uint64_t om_compr)
+                      const ss_buffers *bufs, bool column)
 {
     ms_colv v;
     MS_TRY(colv_of(in, v));
     if (v.g.kind == MS_BLOCKWISE_INDIVIDUAL) {
         if (bufs) return ms_fail(MS_ERR_INVALID, "blockwise_individual_f: select_sum needs temporaries of its own");
         MS_TRY(launch_bwi_select_sum(in, p, d_result, accumulate, s));
-        if (om) hipLaunchKernelGGL(k_set_meta_one, dim3(1), dim3(1), 0, s, om, om_compr);
+        if (column) hipLaunchKernelGGL(k_set_meta_one, dim3(1), dim3(1), 0, s, d_result, v.g.kind);
         MS_HIP(hipGetLastError());
         return MS_OK;
     }
@@ -901,8 +902,8 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
     const bool single = ends && nb <= (by_value ? SS_SINGLE_GENERIC : SS_SINGLE);
     uint64_t *part = single ? nullptr : bufs ? bufs->part : (uint64_t *)sc.get(SS_MAX_PARTS * 8);
     if (!part && !single) return ms_fail(MS_ERR_NOMEM, "select_sum scratch");
-    const int rest = v.g.kind != MS_UNCOMPR && v.g.kind != MS_RLE;
-    const ss_end end = {part, single ? d_result : nullptr, om, om_compr, rest};
+    const ss_end meta = column ? SS_META : 0;
+    const ss_end end = single ? (uint64_t)d_result | SS_RESULT | meta : (uint64_t)part;
     switch (v.g.kind) {
     case MS_UNCOMPR:
         grid = grid_for(nb, WG * 32ull, 2048);
@@ -978,8 +979,8 @@ int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bo
     MS_HIP(hipGetLastError());
     if (single) return MS_OK;
     static_assert(SS_MAX_PARTS >= 8192, "every grid above is capped at 8192 workgroups");
-    hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(WG), 0, s, v, p, (const uint64_t *)part, grid, with_rest, d_result,
-                       om, om_compr);
+    hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(WG), 0, s, v, p, (const uint64_t *)part, grid, with_rest,
+                       (uint64_t)d_result | meta);
     MS_HIP(hipGetLastError());
     return MS_OK;
 }

@@ -44,6 +44,10 @@ void release_kept();
 // device holds at once, queried once per kernel.
 uint32_t resident_grid(const void *kernel, uint32_t wg);
 
+// Bytes of a column's meta at the start of its allocation; index,
+// references and view table, where it has them, and its image follow.
+constexpr uint64_t COL_META_BYTES = 256;
+
 // decode side -------------------------------------------------------
 int launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t s);
 // Caller-provided device buffers of launch_select_sum: `part` holds
@@ -58,10 +62,10 @@ struct ss_buffers {
 };
 // *d_result (+)= sum of x_i with pred(x_i); the result is zeroed first
 // unless `accumulate`.  With `bufs` no device memory is allocated.
-// With `om` the result also sets the meta of the uncompr_f column d_result
-// is the one value of (count 1, `om_compr` compressed bytes).
+// `column`: d_result is the value of a one-value uncompr_f column, whose
+// meta (in front of it) is set too.
 int launch_select_sum(const ms_col *in, const ms_pred &p, uint64_t *d_result, bool accumulate, hipStream_t s,
-                      const ss_buffers *bufs = nullptr, ms_dev_meta *om = nullptr, uint64_t om_compr = 0);
+                      const ss_buffers *bufs = nullptr, bool column = false);
 // writes the column's `count` values to d_out (uncompressed); with `om`
 // also the whole meta of the uncompr_f column d_out belongs to
 int launch_decompress(const ms_col *in, uint64_t *d_out, hipStream_t s, ms_dev_meta *om = nullptr);
