@@ -1,10 +1,7 @@
 // ms_abi.hip -- the C-ABI of include/morphstore_hip.h: column management
 // and operator orchestration.  Entry points never throw; errors are status
 // codes with a per-thread message (ms_last_error).
-#include <list>
-#include <map>
 #include <mutex>
-#include <unordered_map>
 #include <unordered_set>
 #include <stdarg.h>
 #include <stdio.h>
@@ -13,6 +10,7 @@
 #include <string>
 #include <vector>
 
+#include "ms_kept.hpp"
 #include "ms_kernels.h"
 
 static thread_local std::string g_err;
@@ -87,146 +85,67 @@ int plan_hold(void (*release)(void *), void *obj)
 }
 
 // ------------------------------------------------------------------
-// Memory of the null stream, kept for its next call.  hipMallocAsync's pool
-// gives memory back to the system on a free whatever its release threshold
-// says, so that every call maps and unmaps its buffers again: of the
-// select, project and agg_sum over 2^24 values (0.31 ms of kernels) that
-// was 0.8 to 12 ms, growing with the memory the process holds.  A block
-// freed on the null stream is handed to a later call on the null stream
-// without waiting: the stream orders its uses, and unlike a created
-// stream it is never destroyed and never captured; other streams keep
-// using hipMallocAsync.  At most a sixteenth of the device's memory is
-// kept (the least recently freed blocks go first), all of it is given back
-// when an allocation of the library fails and when the last column is freed.
+// Memory of the null stream, kept for its next call (ms_kept.hpp).  All of it
+// is given back when an allocation of the library fails and when the last
+// column is freed.
 // ------------------------------------------------------------------
 namespace {
 
-struct null_cache {
-    struct block {
-        void *p;
-        size_t bytes;
-        int dev;
-    };
-    typedef std::list<block> lru;                       // free blocks, least recently freed first
-    std::mutex mu;
-    std::unordered_map<void *, block> live;             // blocks in use
-    lru free_;
-    std::map<std::pair<int, size_t>, std::vector<lru::iterator>> by_size;   // (device, bytes)
-    size_t kept = 0, limit = 0;
-
-    // Sizes are rounded so that calls of nearly the same sizes share
-    // blocks: eighths of a power of two, at most 32 MiB.
-    static size_t round_size(size_t n)
+// The device `dev` for the calling thread, for as long as the object lives.
+struct on_device {
+    int before = -1;
+    explicit on_device(int dev)
     {
-        size_t step = 256;
-        while (step * 16 <= n && step < (32u << 20)) step *= 2;
-        return (n + step - 1) / step * step;
+        if (hipGetDevice(&before) != hipSuccess || before == dev || hipSetDevice(dev) != hipSuccess) before = -1;
     }
-
-    void unlink(lru::iterator it)
+    ~on_device()
     {
-        auto b = by_size.find({it->dev, it->bytes});
-        for (auto k = b->second.begin(); k != b->second.end(); ++k)
-            if (*k == it) {
-                b->second.erase(k);
-                break;
-            }
-        if (b->second.empty()) by_size.erase(b);
-        kept -= it->bytes;
-        free_.erase(it);
-    }
-
-    void trim(size_t to)
-    {
-        while (kept > to && !free_.empty()) {
-            void *p = free_.front().p;
-            unlink(free_.begin());
-            (void)hipFreeAsync(p, nullptr);
-        }
-    }
-
-    // Everything kept, to the system (waits for the device).
-    void give_back()
-    {
-        if (free_.empty()) return;
-        trim(0);
-        int dev = 0;
-        hipMemPool_t pool;
-        (void)hipDeviceSynchronize();
-        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
-            (void)hipMemPoolTrimTo(pool, 0);
-    }
-
-    void *get(size_t bytes)
-    {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return nullptr;
-        const size_t want = round_size(bytes);
-        std::lock_guard<std::mutex> lk(mu);
-        // the smallest block that fits, unless it is much too large
-        auto b = by_size.lower_bound({dev, want});
-        if (b != by_size.end() && b->first.first == dev && b->first.second <= want + want / 4) {
-            const lru::iterator it = b->second.back();
-            const block k = *it;
-            unlink(it);
-            live[k.p] = k;
-            return k.p;
-        }
-        block k = {nullptr, want, dev};
-        if (hipMallocAsync(&k.p, want, nullptr) != hipSuccess) {
-            (void)hipGetLastError();
-            give_back();
-            k.bytes = bytes;
-            if (hipMallocAsync(&k.p, bytes, nullptr) != hipSuccess) return nullptr;
-        }
-        live[k.p] = k;
-        return k.p;
-    }
-
-    // false: not one of this cache's blocks
-    bool put(void *p)
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        auto l = live.find(p);
-        if (l == live.end()) return false;
-        const block k = l->second;
-        live.erase(l);
-        if (!limit) {
-            size_t avail = 0, total = 0;
-            limit = hipMemGetInfo(&avail, &total) == hipSuccess && total ? total / 16 : 1u << 30;
-        }
-        if (k.bytes > limit) {
-            (void)hipFreeAsync(p, nullptr);
-            return true;
-        }
-        free_.push_back(k);
-        by_size[{k.dev, k.bytes}].push_back(std::prev(free_.end()));
-        kept += k.bytes;
-        trim(limit);
-        return true;
-    }
-
-
-    void drop()
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        trim(0);
+        if (before >= 0) (void)hipSetDevice(before);
     }
 };
 
-null_cache &cache()
+struct null_stream {
+    static int device()
+    {
+        int dev = -1;
+        return hipGetDevice(&dev) == hipSuccess ? dev : -1;
+    }
+    static void *alloc(int, size_t bytes)   // of the current device
+    {
+        void *p = nullptr;
+        if (hipMallocAsync(&p, bytes, nullptr) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static void free(int dev, void *p)
+    {
+        const on_device on(dev);
+        (void)hipFreeAsync(p, nullptr);
+    }
+    static void settle(int dev)
+    {
+        const on_device on(dev);
+        hipMemPool_t pool;
+        (void)hipDeviceSynchronize();
+        if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    }
+    static size_t total(int dev)
+    {
+        const on_device on(dev);
+        size_t avail = 0, total = 0;
+        return hipMemGetInfo(&avail, &total) == hipSuccess ? total : 0;
+    }
+};
+
+kept_memory<null_stream> &cache()
 {
-    static null_cache *c = new null_cache();   // outlives every static object's destructor
+    static kept_memory<null_stream> *c = new kept_memory<null_stream>();   // outlives every static object's destructor
     return *c;
 }
 
 }  // namespace
 
-void release_kept()
-{
-    std::lock_guard<std::mutex> lk(cache().mu);
-    cache().give_back();
-}
+void release_kept() { cache().release(); }
 
 // Frees memory of dev_alloc (or of a created stream) in order on s.
 static void free_ordered(void *p, hipStream_t s)

@@ -1,0 +1,156 @@
+// ms_kept.hpp -- device memory of the null stream, kept for its next call.
+//
+// hipMallocAsync's pool gives memory back to the system on a free whatever
+// its release threshold says, so that every call maps and unmaps its buffers
+// again: of the select, project and agg_sum over 2^24 values (0.31 ms of
+// kernels) that was 0.8 to 12 ms, growing with the memory the process holds.
+// A block freed on the null stream is handed to a later call on the null
+// stream without waiting: the stream orders its uses, and unlike a created
+// stream it is never destroyed and never captured; other streams keep
+// using hipMallocAsync.  At most a sixteenth of a device's memory is kept (the
+// least recently freed blocks go first).
+//
+// The rules only: `Api` is the device's side, so that they can be checked on
+// the host.  It has static device() (the current one), alloc(device, bytes),
+// free(device, p), settle(device) (waits for the device and gives its unused
+// memory to the system) and total(device) (its bytes).
+#pragma once
+
+#include <stddef.h>
+
+#include <list>
+#include <map>
+#include <mutex>
+#include <unordered_map>
+#include <utility>
+#include <vector>
+
+namespace ms {
+
+template <class Api>
+class kept_memory {
+    struct block {
+        void *p;
+        size_t bytes;
+        int dev;
+    };
+    typedef std::list<block> lru;                            // free blocks, least recently freed first
+    struct device {
+        lru free_;
+        std::map<size_t, std::vector<typename lru::iterator>> by_size;
+        size_t kept = 0, limit = 0;
+    };
+    static constexpr int MAX_DEVICES = 64;
+
+    std::mutex mu;
+    std::unordered_map<void *, block> live;                  // blocks in use
+    device devs[MAX_DEVICES];
+
+    // Sizes are rounded so that calls of nearly the same sizes share
+    // blocks: eighths of a power of two, at most 32 MiB.
+    static size_t round_size(size_t n)
+    {
+        size_t step = 256;
+        while (step * 16 <= n && step < (32u << 20)) step *= 2;
+        return (n + step - 1) / step * step;
+    }
+
+    static void unlink(device &d, typename lru::iterator it)
+    {
+        auto b = d.by_size.find(it->bytes);
+        for (auto k = b->second.begin(); k != b->second.end(); ++k)
+            if (*k == it) {
+                b->second.erase(k);
+                break;
+            }
+        if (b->second.empty()) d.by_size.erase(b);
+        d.kept -= it->bytes;
+        d.free_.erase(it);
+    }
+
+    static void trim(device &d, size_t to)
+    {
+        while (d.kept > to && !d.free_.empty()) {
+            const block k = d.free_.front();
+            unlink(d, d.free_.begin());
+            Api::free(k.dev, k.p);
+        }
+    }
+
+    void give_back(int dev)
+    {
+        if (devs[dev].free_.empty()) return;
+        trim(devs[dev], 0);
+        Api::settle(dev);
+    }
+
+public:
+    // Memory of the current device for a call on the null stream.
+    void *get(size_t bytes)
+    {
+        const int dev = Api::device();
+        if (dev < 0 || dev >= MAX_DEVICES) return nullptr;
+        const size_t want = round_size(bytes);
+        std::lock_guard<std::mutex> lk(mu);
+        device &d = devs[dev];
+        // the smallest block that fits, unless it is much too large
+        auto b = d.by_size.lower_bound(want);
+        if (b != d.by_size.end() && b->first <= want + want / 4) {
+            const auto it = b->second.back();
+            const block k = *it;
+            unlink(d, it);
+            live[k.p] = k;
+            return k.p;
+        }
+        block k = {Api::alloc(dev, want), want, dev};
+        if (!k.p) {
+            give_back(dev);
+            k.bytes = bytes;
+            k.p = Api::alloc(dev, bytes);
+            if (!k.p) return nullptr;
+        }
+        live[k.p] = k;
+        return k.p;
+    }
+
+    // Takes back memory of get(), whatever device is current.  false: not a
+    // block of this object.
+    bool put(void *p)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto l = live.find(p);
+        if (l == live.end()) return false;
+        const block k = l->second;
+        live.erase(l);
+        device &d = devs[k.dev];
+        if (!d.limit) {
+            const size_t total = Api::total(k.dev);
+            d.limit = total ? total / 16 : 1u << 30;
+        }
+        if (k.bytes > d.limit) {
+            Api::free(k.dev, p);
+            return true;
+        }
+        d.free_.push_back(k);
+        d.by_size[k.bytes].push_back(std::prev(d.free_.end()));
+        d.kept += k.bytes;
+        trim(d, d.limit);
+        return true;
+    }
+
+    // Frees every block that is not in use.
+    void drop()
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (device &d : devs) trim(d, 0);
+    }
+
+    // The same, and everything unused goes to the system.
+    void release()
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (int dev = 0; dev < MAX_DEVICES; dev++) give_back(dev);
+    }
+};
+
+}  // namespace ms
