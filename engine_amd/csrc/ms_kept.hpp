@@ -18,12 +18,13 @@
 
 #include <stddef.h>
 
+#include <deque>
+#include <iterator>
 #include <list>
 #include <map>
 #include <mutex>
 #include <unordered_map>
 #include <utility>
-#include <vector>
 
 namespace ms {
 
@@ -37,7 +38,9 @@ class kept_memory {
     typedef std::list<block> lru;                            // free blocks, least recently freed first
     struct device {
         lru free_;
-        std::map<size_t, std::vector<typename lru::iterator>> by_size;
+        // blocks of each size, least recently freed first as well: get()
+        // takes a class's last one, trim() the first of the one it is in
+        std::map<size_t, std::deque<typename lru::iterator>> by_size;
         size_t kept = 0, limit = 0;
     };
     static constexpr int MAX_DEVICES = 64;
@@ -55,24 +58,25 @@ class kept_memory {
         return (n + step - 1) / step * step;
     }
 
-    static void unlink(device &d, typename lru::iterator it)
+    typedef typename std::map<size_t, std::deque<typename lru::iterator>>::iterator size_class;
+
+    // Takes the last or the first block of a size class out of the lists.
+    static block take(device &d, size_class b, bool last)
     {
-        auto b = d.by_size.find(it->bytes);
-        for (auto k = b->second.begin(); k != b->second.end(); ++k)
-            if (*k == it) {
-                b->second.erase(k);
-                break;
-            }
+        const auto it = last ? b->second.back() : b->second.front();
+        const block k = *it;
+        if (last) b->second.pop_back();
+        else b->second.pop_front();
         if (b->second.empty()) d.by_size.erase(b);
-        d.kept -= it->bytes;
+        d.kept -= k.bytes;
         d.free_.erase(it);
+        return k;
     }
 
     static void trim(device &d, size_t to)
     {
         while (d.kept > to && !d.free_.empty()) {
-            const block k = d.free_.front();
-            unlink(d, d.free_.begin());
+            const block k = take(d, d.by_size.find(d.free_.front().bytes), false);
             Api::free(k.dev, k.p);
         }
     }
@@ -96,9 +100,7 @@ public:
         // the smallest block that fits, unless it is much too large
         auto b = d.by_size.lower_bound(want);
         if (b != d.by_size.end() && b->first <= want + want / 4) {
-            const auto it = b->second.back();
-            const block k = *it;
-            unlink(d, it);
+            const block k = take(d, b, true);
             live[k.p] = k;
             return k.p;
         }

@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <map>
+#include <vector>
 
 #include "ms_kept.hpp"
 
@@ -135,10 +136,26 @@ static void devices(kept &k)
     CHECK(fake::used[0] == 0);
 }
 
+// Finding and freeing a block takes no longer the more of its size are free.
+static void many(kept &k)
+{
+    const int n = 500000;
+    fake::size = (size_t)n * 4096 * 32;
+    std::vector<void *> p(n);
+    for (int i = 0; i < n; i++) p[i] = k.get(1000);
+    for (int i = 0; i < n; i++) CHECK(k.put(p[i]));
+    CHECK(fake::frees == 0);
+    for (int i = 0; i < n; i++) CHECK(k.get(1000) == p[n - 1 - i]);   // the latest first
+    for (int i = 0; i < n; i++) CHECK(k.put(p[i]));
+    k.drop();
+    CHECK(fake::frees == n);
+}
+
 int main(int argc, char **argv)
 {
     const std::pair<const char *, void (*)(kept &)> checks[] = {
-        {"reuse", reuse}, {"limit", limit}, {"failure", failure}, {"drop", drop}, {"devices", devices}};
+        {"reuse", reuse}, {"limit", limit}, {"failure", failure}, {"drop", drop}, {"devices", devices},
+        {"many", many}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.first)) {
             kept k;
