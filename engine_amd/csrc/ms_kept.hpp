@@ -17,6 +17,7 @@
 #pragma once
 
 #include <stddef.h>
+#include <stdint.h>
 
 #include <deque>
 #include <iterator>
@@ -34,6 +35,7 @@ class kept_memory {
         void *p;
         size_t bytes;
         int dev;
+        size_t over;   // bytes more than its use asks for
     };
     typedef std::list<block> lru;                            // free blocks, least recently freed first
     struct device {
@@ -41,21 +43,25 @@ class kept_memory {
         // blocks of each size, least recently freed first as well: get()
         // takes a class's last one, trim() the first of the one it is in
         std::map<size_t, std::deque<typename lru::iterator>> by_size;
-        size_t kept = 0, limit = 0;
+        size_t kept = 0, limit = 0, over = 0;   // over: of all blocks in use
     };
     static constexpr int MAX_DEVICES = 64;
+    // A block may be a quarter larger than asked for, but a column holds it
+    // for as long as it lives: all blocks in use together are at most this
+    // much too large.
+    static constexpr size_t MAX_OVER = 64u << 20;
 
     std::mutex mu;
     std::unordered_map<void *, block> live;                  // blocks in use
     device devs[MAX_DEVICES];
 
-    // Sizes are rounded so that calls of nearly the same sizes share
-    // blocks: eighths of a power of two, at most 32 MiB.
+    // Sizes are rounded up to what the pool takes from the system for them
+    // anyway (pages of 4 KiB up to 1 MiB, of 2 MiB above), so that calls of
+    // nearly the same sizes share blocks and no memory is lost.
     static size_t round_size(size_t n)
     {
-        size_t step = 256;
-        while (step * 16 <= n && step < (32u << 20)) step *= 2;
-        return (n + step - 1) / step * step;
+        const size_t page = n <= (1u << 20) ? 4096 : 2u << 20;
+        return n > SIZE_MAX - page ? n : (n + page - 1) / page * page;
     }
 
     typedef typename std::map<size_t, std::deque<typename lru::iterator>>::iterator size_class;
@@ -97,18 +103,19 @@ public:
         const size_t want = round_size(bytes);
         std::lock_guard<std::mutex> lk(mu);
         device &d = devs[dev];
-        // the smallest block that fits, unless it is much too large
+        // the smallest block that fits, unless it is too large
         auto b = d.by_size.lower_bound(want);
-        if (b != d.by_size.end() && b->first <= want + want / 4) {
-            const block k = take(d, b, true);
+        if (b != d.by_size.end() && b->first - want <= want / 4 && d.over + (b->first - want) <= MAX_OVER) {
+            block k = take(d, b, true);
+            k.over = k.bytes - want;
+            d.over += k.over;
             live[k.p] = k;
             return k.p;
         }
-        block k = {Api::alloc(dev, want), want, dev};
+        block k = {Api::alloc(dev, want), want, dev, 0};
         if (!k.p) {
             give_back(dev);
-            k.bytes = bytes;
-            k.p = Api::alloc(dev, bytes);
+            k.p = Api::alloc(dev, want);
             if (!k.p) return nullptr;
         }
         live[k.p] = k;
@@ -125,6 +132,7 @@ public:
         const block k = l->second;
         live.erase(l);
         device &d = devs[k.dev];
+        d.over -= k.over;
         if (!d.limit) {
             const size_t total = Api::total(k.dev);
             d.limit = total ? total / 16 : 1u << 30;

@@ -151,11 +151,41 @@ static void many(kept &k)
     CHECK(fake::frees == n);
 }
 
+// What fits without the cache fits with it: a block is larger than asked for
+// by less than the pool's page, and larger ones are reused within a budget.
+static void excess(kept &k)
+{
+    for (size_t n : {(size_t)1, (size_t)4096, (size_t)5000, MiB, MiB + 1, 3 * MiB + 256, 33 * MiB + 256, 700 * MiB + 1}) {
+        void *p = k.get(n);
+        CHECK(p && fake::held[p].bytes >= n && fake::held[p].bytes - n < (n <= MiB ? 4096 : 2 * MiB));
+        CHECK(k.put(p));
+        k.drop();
+    }
+    void *a = k.get(901 * MiB), *b = k.get(121 * MiB);
+    CHECK(a && b && k.put(a) && k.put(b));
+    k.drop();
+    CHECK(k.get(SIZE_MAX - 100) == nullptr && k.get(SIZE_MAX) == nullptr);
+
+    fake::size = 64 * 1024 * MiB;             // 4 GiB are kept
+    kept l;
+    void *p[10], *q[10];
+    for (void *&x : p) x = l.get(120 * MiB);
+    for (void *x : p) CHECK(l.put(x));
+    for (int i = 0; i < 10; i++) {
+        q[i] = l.get(100 * MiB);              // 20 MiB too large, three times
+        CHECK((fake::held[q[i]].bytes == 120 * MiB) == (i < 3));
+    }
+    CHECK(l.put(q[1]));
+    void *r = l.get(101 * MiB);               // the budget is free again
+    CHECK(fake::held[r].bytes == 120 * MiB);
+    CHECK(l.get(80 * MiB) && fake::held.size() == 10 + 7 + 1);   // 40 MiB too large: never
+}
+
 int main(int argc, char **argv)
 {
     const std::pair<const char *, void (*)(kept &)> checks[] = {
         {"reuse", reuse}, {"limit", limit}, {"failure", failure}, {"drop", drop}, {"devices", devices},
-        {"many", many}};
+        {"many", many}, {"excess", excess}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.first)) {
             kept k;
