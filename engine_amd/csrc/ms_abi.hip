@@ -139,7 +139,9 @@ struct null_stream {
 
 kept_memory<null_stream> &cache()
 {
-    static kept_memory<null_stream> *c = new kept_memory<null_stream>();   // outlives every static object's destructor
+    // never destroyed: columns are freed after every static object's destructor
+    alignas(kept_memory<null_stream>) static unsigned char place[sizeof(kept_memory<null_stream>)];
+    static kept_memory<null_stream> *c = new (place) kept_memory<null_stream>();
     return *c;
 }
 

@@ -10,6 +10,8 @@
 // using hipMallocAsync.  At most a sixteenth of a device's memory is kept (the
 // least recently freed blocks go first).
 //
+// Nothing here throws: the entry points that allocate are C.
+//
 // The rules only: `Api` is the device's side, so that they can be checked on
 // the host.  It has static device() (the current one), alloc(device, bytes),
 // free(device, p), settle(device) (waits for the device and gives its unused
@@ -94,6 +96,18 @@ class kept_memory {
         Api::settle(dev);
     }
 
+    // Notes a block in use and gives its address.  Without host memory for
+    // that the caller has it all the same: put() then does not know it.
+    void *hold(const block &k)
+    {
+        try {
+            live.emplace(k.p, k);
+        } catch (...) {
+            devs[k.dev].over -= k.over;
+        }
+        return k.p;
+    }
+
 public:
     // Memory of the current device for a call on the null stream.
     void *get(size_t bytes)
@@ -109,8 +123,7 @@ public:
             block k = take(d, b, true);
             k.over = k.bytes - want;
             d.over += k.over;
-            live[k.p] = k;
-            return k.p;
+            return hold(k);
         }
         block k = {Api::alloc(dev, want), want, dev, 0};
         if (!k.p) {
@@ -118,8 +131,7 @@ public:
             k.p = Api::alloc(dev, want);
             if (!k.p) return nullptr;
         }
-        live[k.p] = k;
-        return k.p;
+        return hold(k);
     }
 
     // Takes back memory of get(), whatever device is current.  false: not a
@@ -141,8 +153,20 @@ public:
             Api::free(k.dev, p);
             return true;
         }
-        d.free_.push_back(k);
-        d.by_size[k.bytes].push_back(std::prev(d.free_.end()));
+        try {
+            d.free_.push_back(k);
+            try {
+                d.by_size[k.bytes].push_back(std::prev(d.free_.end()));
+            } catch (...) {
+                const auto b = d.by_size.find(k.bytes);
+                if (b != d.by_size.end() && b->second.empty()) d.by_size.erase(b);
+                d.free_.pop_back();
+                throw;
+            }
+        } catch (...) {   // no host memory to keep it with
+            Api::free(k.dev, p);
+            return true;
+        }
         d.kept += k.bytes;
         trim(d, d.limit);
         return true;

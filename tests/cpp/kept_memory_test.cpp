@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <map>
+#include <new>
 #include <vector>
 
 #include "ms_kept.hpp"
@@ -19,6 +20,26 @@
     } while (0)
 
 static const size_t MiB = 1u << 20;
+
+// operator new fails from the g_news-th call on, for g_fails calls.
+static long g_news = -1, g_fails = 0;
+__attribute__((noinline)) void *operator new(size_t n)
+{
+    if (g_news == 0 && g_fails > 0) {
+        g_fails--;
+        throw std::bad_alloc();
+    }
+    if (g_news > 0) g_news--;
+    if (void *p = malloc(n)) return p;
+    throw std::bad_alloc();
+}
+__attribute__((noinline)) void operator delete(void *p) noexcept { free(p); }
+__attribute__((noinline)) void operator delete(void *p, size_t) noexcept { free(p); }
+struct host_memory_back {                     // for the test's own bookkeeping
+    long news = g_news;
+    host_memory_back() { g_news = -1; }
+    ~host_memory_back() { g_news = news; }
+};
 
 // Two devices of `size` bytes; an allocation is a key of `held`.
 struct fake {
@@ -34,6 +55,7 @@ struct fake {
     static int device() { return current; }
     static void *alloc(int dev, size_t bytes)
     {
+        const host_memory_back ours;
         CHECK(dev == current && bytes);
         if (used[dev] + bytes > size) return nullptr;
         void *p = (void *)next;
@@ -181,11 +203,41 @@ static void excess(kept &k)
     CHECK(l.get(80 * MiB) && fake::held.size() == 10 + 7 + 1);   // 40 MiB too large: never
 }
 
+// Without host memory calls are served and nothing is lost or freed twice:
+// one to three allocations of the host fail at every point of a few calls.
+static void host_memory(kept &)
+{
+    for (long fails = 1; fails <= 3; fails++)
+        for (long at = 0; at < 40; at++) {
+            kept k;
+            void *p[6];
+            for (int round = 0; round < 3; round++) {
+                if (round == 1) {
+                    g_news = at;
+                    g_fails = fails;
+                }
+                for (int i = 0; i < 6; i++) {
+                    p[i] = k.get((1 + i / 2) * 8192);
+                    CHECK(p[i] && fake::held.count(p[i]));
+                    for (int j = 0; j < i; j++) CHECK(p[j] != p[i]);
+                }
+                for (int i = 0; i < 6; i++)
+                    if (!k.put(p[i])) fake::free(0, p[i]);   // as the caller does
+            }
+            g_news = -1;
+            CHECK(k.get(8192));
+            k.drop();
+            CHECK(fake::held.size() == 1);
+            fake::free(0, fake::held.begin()->first);
+        }
+}
+
 int main(int argc, char **argv)
 {
     const std::pair<const char *, void (*)(kept &)> checks[] = {
         {"reuse", reuse}, {"limit", limit}, {"failure", failure}, {"drop", drop}, {"devices", devices},
-        {"many", many}, {"excess", excess}};
+        {"many", many}, {"excess", excess},
+        {"host_memory", host_memory}};
     for (const auto &c : checks)
         if (argc > 1 && !strcmp(argv[1], c.first)) {
             kept k;

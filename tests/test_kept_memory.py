@@ -1,7 +1,7 @@
 """The rules of the null stream's kept memory, compiled for the host: reuse,
 the limit and the order in which blocks go, give-back on failure, the drop,
-blocks of several devices, many free blocks of one size, and how much larger
-than asked for a block may be."""
+blocks of several devices, many free blocks of one size, how much larger
+than asked for a block may be, and calls without host memory."""
 import os
 import subprocess
 
@@ -20,7 +20,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["reuse", "limit", "failure", "drop", "devices", "many", "excess"])
+@pytest.mark.parametrize("check", ["reuse", "limit", "failure", "drop", "devices", "many", "excess", "host_memory"])
 def test_kept_memory(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
