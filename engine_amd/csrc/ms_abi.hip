@@ -63,16 +63,6 @@ static thread_local ms_plan *g_rec = nullptr;
 
 static uint64_t round256(uint64_t x) { return (x + 255) / 256 * 256; }
 
-// hipMalloc, with the kept memory of the null stream given back if it fails.
-static hipError_t malloc_arena(uint8_t **p, size_t bytes)
-{
-    hipError_t e = hipMalloc((void **)p, bytes);
-    if (e == hipSuccess) return e;
-    (void)hipGetLastError();
-    ms::release_kept();
-    return hipMalloc((void **)p, bytes);
-}
-
 namespace ms {
 
 bool plan_capturing() { return g_rec && g_rec->recording && g_rec->mode == 1; }
@@ -149,6 +139,34 @@ kept_memory<null_stream> &cache()
 
 void release_kept() { cache().release(); }
 
+template <class Malloc>
+static hipError_t retried(hipStream_t s, const Malloc &m)
+{
+    hipError_t e = m();
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    // giving back waits for the device, which a capture does not allow
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s && (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)) {
+        (void)hipGetLastError();
+        return e;
+    }
+    release_kept();
+    e = m();
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    return retried(nullptr, [&] { return hipMalloc(p, bytes); });
+}
+
+hipError_t device_malloc_async(void **p, size_t bytes, hipStream_t s)
+{
+    return retried(s, [&] { return hipMallocAsync(p, bytes, s); });
+}
+
 // Frees memory of dev_alloc (or of a created stream) in order on s.
 static void free_ordered(void *p, hipStream_t s)
 {
@@ -166,11 +184,7 @@ void *dev_alloc(size_t bytes, hipStream_t s)
     }
     void *p = nullptr;
     if (s == nullptr) p = cache().get(bytes);
-    else if (hipMallocAsync(&p, bytes, s) != hipSuccess) {
-        (void)hipGetLastError();
-        release_kept();
-        if (hipMallocAsync(&p, bytes, s) != hipSuccess) return nullptr;
-    }
+    else if (device_malloc_async(&p, bytes, s) != hipSuccess) return nullptr;
     if (!p) return nullptr;
     if (g_rec && g_rec->recording && g_rec->mode == 0) g_rec->measured += bytes;
     return p;
@@ -921,7 +935,7 @@ extern "C" int ms_plan_create(ms_plan **out, uint64_t arena_bytes)
     if (!p) return ms_fail(MS_ERR_NOMEM, "host allocation");
     p->arena_bytes = arena_bytes;
     p->mode = arena_bytes ? 1 : 0;
-    if (arena_bytes && malloc_arena(&p->arena, arena_bytes) != hipSuccess) {
+    if (arena_bytes && device_malloc((void **)&p->arena, arena_bytes) != hipSuccess) {
         delete p;
         return ms_fail(MS_ERR_NOMEM, "plan arena of %llu bytes", (unsigned long long)arena_bytes);
     }
@@ -936,7 +950,7 @@ extern "C" int ms_plan_begin(ms_plan *p, void *stream)
     if (p->mode == 0 && p->measured) {
         // the measuring pass is done: allocate the arena and capture
         p->arena_bytes = p->measured + (1u << 20);
-        if (malloc_arena(&p->arena, p->arena_bytes) != hipSuccess)
+        if (device_malloc((void **)&p->arena, p->arena_bytes) != hipSuccess)
             return ms_fail(MS_ERR_NOMEM, "plan arena of %llu bytes", (unsigned long long)p->arena_bytes);
         p->mode = 1;
     }

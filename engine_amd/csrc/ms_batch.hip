@@ -409,12 +409,7 @@ static int ensure(T **p, size_t &cap, size_t n)
     if (*p) MS_HIP(hipFree(*p));
     *p = nullptr;
     cap = 0;
-    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-    if (hipMalloc((void **)p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        release_kept();
-        MS_HIP(hipMalloc((void **)p, bytes));
-    }
+    MS_HIP(device_malloc((void **)p, std::max<size_t>(n, 1) * sizeof(T)));
     cap = std::max<size_t>(n, 1);
     return MS_OK;
 }
@@ -545,7 +540,7 @@ static int build(ms_batch *b, hipStream_t s)
     if (!b->have_meta) {
         MS_HIP(hipMemcpyAsync(b->dE, b->E.data(), nE * sizeof(ms_bentry), hipMemcpyHostToDevice, s));
         ms_col_meta *dm = nullptr;
-        MS_HIP(hipMallocAsync((void **)&dm, std::max<size_t>(nE, 1) * sizeof(ms_col_meta), s));
+        MS_HIP(device_malloc_async((void **)&dm, std::max<size_t>(nE, 1) * sizeof(ms_col_meta), s));
         if (nE) hipLaunchKernelGGL(k_batch_meta, dim3((nE + 255) / 256), dim3(256), 0, s, b->dE, (uint64_t)nE, dm);
         MS_HIP(hipGetLastError());
         b->meta.resize(nE);
@@ -767,7 +762,7 @@ extern "C" int ms_batch_view_times(ms_batch *b, uint64_t *d_results, uint32_t re
     MS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     if (khz <= 0) return ms_fail(MS_ERR_HIP, "no wall clock rate");
     unsigned long long *ticks = nullptr;
-    MS_HIP(hipMallocAsync((void **)&ticks, std::max<uint64_t>(b->ntags, 1) * 8, s));
+    MS_HIP(device_malloc_async((void **)&ticks, std::max<uint64_t>(b->ntags, 1) * 8, s));
     int rc = launch_fill_u64((uint64_t *)ticks, std::max<uint64_t>(b->ntags, 1), 0, s);
     for (uint32_t r = 0; r < reps && !rc; r++) {
         hipLaunchKernelGGL(k_batch_select_sum_timed, dim3(b->grid), dim3(WG), 0, s, (const ms_bentry *)b->dE,

@@ -36,9 +36,14 @@ int plan_hold(void (*release)(void *), void *obj);
 // device memory of the operators (from a recording plan's arena if any)
 void *dev_alloc(size_t bytes, hipStream_t s);
 void dev_free(void *p, hipStream_t s);
-// gives back the memory that dev_alloc keeps for the null stream (for a
-// direct allocation that failed; waits for the device)
+// gives back the memory that dev_alloc keeps for the null stream (waits for
+// the device)
 void release_kept();
+// hipMalloc and hipMallocAsync; one that fails is tried again with that
+// memory given back, and no error is left for the next hipGetLastError.
+// Every allocation of the library goes through these two or dev_alloc.
+hipError_t device_malloc(void **p, size_t bytes);
+hipError_t device_malloc_async(void **p, size_t bytes, hipStream_t s);
 
 // Workgroups of `kernel` (wg threads, no dynamic LDS) that the current
 // device holds at once, queried once per kernel.

@@ -635,8 +635,9 @@ extern "C" int ms_mlp_create(ms_mlp **out, uint64_t seed)
     if (!out) return ms_fail(MS_ERR_INVALID, "null argument");
     ms_mlp *m = new (std::nothrow) ms_mlp();
     if (!m) return ms_fail(MS_ERR_NOMEM, "host allocation");
-    if (hipMalloc((void **)&m->prm, NPARAM * 4) != hipSuccess || hipMalloc((void **)&m->m1, NPARAM * 4) != hipSuccess ||
-        hipMalloc((void **)&m->m2, NPARAM * 4) != hipSuccess) {
+    if (device_malloc((void **)&m->prm, NPARAM * 4) != hipSuccess ||
+        device_malloc((void **)&m->m1, NPARAM * 4) != hipSuccess ||
+        device_malloc((void **)&m->m2, NPARAM * 4) != hipSuccess) {
         (void)hipFree(m->prm); (void)hipFree(m->m1); (void)hipFree(m->m2);
         delete m;
         return ms_fail(MS_ERR_NOMEM, "mlp parameters");

@@ -2,6 +2,7 @@
 one call's output to another's scratch, columns read on a created stream
 before they are freed, frees from several threads, and frees while a plan
 captures leave every result as it was."""
+import ctypes
 import threading
 
 import numpy as np
@@ -9,7 +10,8 @@ import pytest
 
 import engine_amd as ea
 from engine_amd import datagen, hip
-from engine_amd.formats import MS_CMP_LT, default_delta_dynamic_vbp_f, dynamic_vbp_f, rle_f, uncompr_f
+from engine_amd.formats import (MS_CMP_LT, MS_ERR_NOMEM, default_delta_dynamic_vbp_f, dynamic_vbp_f, rle_f,
+                                uncompr_f)
 
 pytestmark = pytest.mark.gpu
 
@@ -73,3 +75,50 @@ def test_free_while_a_plan_captures():
         assert np.array_equal(again.values(), x ^ np.uint64(1))
     del total
     plan.free()
+
+
+def last_error():
+    return hip.hip().hipGetLastError()
+
+
+def used_by_pool():
+    """Bytes of the null stream's pool that are allocated (kept ones too)."""
+    hip.synchronize()
+    pool, used = ctypes.c_void_p(), ctypes.c_uint64()
+    assert hip.hip().hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+    assert hip.hip().hipMemPoolGetAttribute(pool, 7, ctypes.byref(used)) == 0   # hipMemPoolAttrUsedMemCurrent
+    return used.value
+
+
+@pytest.mark.parametrize("created", [False, True])
+def test_failed_allocation(created):
+    """An allocation that cannot succeed (2^44 values of one run) gives the
+    kept memory back, is an error of its own call and of no later one."""
+    st = hip.Stream() if created else None
+    pair = np.array([7, 1 << 44], np.uint64).view(np.uint8)
+    run = ea.upload_image(rle_f(), pair, 1 << 44, 16, 16)
+    x = datagen.uniform_bits(9, 1 << 20, 20)
+    left = []
+    for _ in range(2):
+        ea.upload_values(x)                   # freed at once: 8 MiB kept
+        kept = used_by_pool()
+        with pytest.raises(ea.MsError) as e:
+            ea.morph(uncompr_f(), run, st)
+        assert e.value.code == MS_ERR_NOMEM
+        assert last_error() == 0
+        left.append(used_by_pool())
+        assert left[-1] <= kept - x.nbytes
+    assert left[0] == left[1]
+    assert np.array_equal(ea.morph(dynamic_vbp_f(512, 2048, 8), ea.upload_values(x), st).values(st), x)
+
+
+def test_failed_plan_arena():
+    x = datagen.uniform_bits(9, 1 << 20, 20)
+    keep = ea.upload_values(x[:10])
+    ea.upload_values(x)
+    kept = used_by_pool()
+    with pytest.raises(ea.MsError) as e:
+        ea.Plan(1 << 46)
+    assert e.value.code == MS_ERR_NOMEM
+    assert last_error() == 0 and used_by_pool() <= kept - x.nbytes
+    assert np.array_equal(keep.values(), x[:10])
