@@ -11,7 +11,7 @@ import os
 import numpy as np
 
 from .formats import BatchConfig, ColMeta, FormatDesc  # noqa: F401
-from .hip import Stream
+from .hip import Stream, device_malloc
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MS_LIB_PATH selects another build of the same library (e.g. a tuning variant)
@@ -26,6 +26,7 @@ _FD, _CM = P(FormatDesc), P(ColMeta)
 _COLP = P(VP)
 ABI = {
     "ms_init": (ctypes.c_int, [ctypes.c_int]),
+    "ms_release_memory": (ctypes.c_int, []),
     "ms_last_error": (ctypes.c_char_p, []),
     "ms_version": (ctypes.c_char_p, []),
     "ms_size_max_byte_any_len": (ctypes.c_int, [_FD, U64, P(U64)]),
@@ -123,6 +124,13 @@ def init(device=0):
     if not _inited:
         check(lib().ms_init(device))
         _inited = True
+
+
+def release_memory():
+    """Returns the device memory that the library keeps for later calls on
+    the null stream to the system (for another allocator of the process)."""
+    init()
+    check(lib().ms_release_memory())
 
 
 class Column:
@@ -302,7 +310,7 @@ class DeviceU64:
         self.n = n
         self.p = VP()
         self._owner = None
-        rc = DeviceU64._hip.hipMalloc(ctypes.byref(self.p), ctypes.c_size_t(8 * n))
+        rc = device_malloc(self.p, 8 * n)
         if rc != 0:
             raise MsError(3, f"hipMalloc failed ({rc})")
 

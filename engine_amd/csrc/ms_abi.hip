@@ -76,8 +76,8 @@ int plan_hold(void (*release)(void *), void *obj)
 
 // ------------------------------------------------------------------
 // Memory of the null stream, kept for its next call (ms_kept.hpp).  All of it
-// is given back when an allocation of the library fails and when the last
-// column is freed.
+// is given back when an allocation of the library fails, when the last
+// column is freed and by ms_release_memory.
 // ------------------------------------------------------------------
 namespace {
 
@@ -364,6 +364,14 @@ extern "C" int ms_init(int device)
 int ms_need_init()
 {
     if (g_device < 0) return ms_fail(MS_ERR_NODEVICE, "ms_init was not called");
+    return MS_OK;
+}
+
+extern "C" int ms_release_memory(void)
+{
+    MS_TRY(ms_need_init());
+    if (plan_capturing()) return ms_fail(MS_ERR_INVALID, "ms_release_memory waits for the device: not in a plan");
+    release_kept();
     return MS_OK;
 }
 

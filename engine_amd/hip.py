@@ -17,6 +17,20 @@ def _ok(rc, what):
         raise RuntimeError(f"{what} failed with hipError {rc}")
 
 
+def device_malloc(p, nbytes):
+    """hipMalloc of nbytes into the c_void_p p; its error code.  One that fails
+    is tried again with the memory that the library keeps given back."""
+    rc = hip().hipMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes))
+    if rc != 0:
+        from . import lib
+        hip().hipGetLastError()
+        if lib().ms_release_memory() == 0:
+            rc = hip().hipMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes))
+            if rc != 0:
+                hip().hipGetLastError()
+    return rc
+
+
 class Event:
     def __init__(self):
         self.e = ctypes.c_void_p()
@@ -93,8 +107,7 @@ class DeviceArray:
         self.dtype = np.dtype(dtype)
         self.n = int(n)
         self.p = ctypes.c_void_p()
-        _ok(hip().hipMalloc(ctypes.byref(self.p), ctypes.c_size_t(max(1, self.n * self.dtype.itemsize))),
-            "hipMalloc")
+        _ok(device_malloc(self.p, max(1, self.n * self.dtype.itemsize)), "hipMalloc")
 
     @classmethod
     def from_numpy(cls, a):

@@ -165,6 +165,13 @@ enum ms_calc_op {
  * allocation pool.  Must be called once per process before anything else. */
 int ms_init(int device);
 
+/* Device memory that calls on the null stream freed is kept for later calls
+ * on it: at most a sixteenth of the device's memory, and none once no column
+ * is alive.  A library allocation that fails gives it back and is tried again;
+ * for another allocator of the process (hipMalloc, torch) this call returns
+ * all of it to the system.  Waits for the device. */
+int ms_release_memory(void);
+
 /* Text of the last error on the calling thread ("" if none). */
 const char *ms_last_error(void);
 

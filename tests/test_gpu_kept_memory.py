@@ -10,8 +10,8 @@ import pytest
 
 import engine_amd as ea
 from engine_amd import datagen, hip
-from engine_amd.formats import (MS_CMP_LT, MS_ERR_NOMEM, default_delta_dynamic_vbp_f, dynamic_vbp_f, rle_f,
-                                uncompr_f)
+from engine_amd.formats import (MS_CMP_LT, MS_ERR_INVALID, MS_ERR_NOMEM, default_delta_dynamic_vbp_f, dynamic_vbp_f,
+                                rle_f, uncompr_f)
 
 pytestmark = pytest.mark.gpu
 
@@ -120,5 +120,45 @@ def test_failed_plan_arena():
     with pytest.raises(ea.MsError) as e:
         ea.Plan(1 << 46)
     assert e.value.code == MS_ERR_NOMEM
+    assert last_error() == 0 and used_by_pool() <= kept - x.nbytes
+    assert np.array_equal(keep.values(), x[:10])
+
+
+def test_release_memory():
+    x = datagen.uniform_bits(9, 1 << 20, 20)
+    keep = ea.upload_values(x[:10])
+    ea.release_memory()
+    before = used_by_pool()
+    ea.upload_values(x)
+    assert used_by_pool() >= before + x.nbytes
+    ea.release_memory()
+    assert used_by_pool() == before
+    assert np.array_equal(keep.values(), x[:10])
+
+
+def test_release_memory_not_while_a_plan_captures():
+    st, plan = hip.Stream(), ea.Plan()
+    col = ea.upload_values(datagen.uniform_bits(9, 5000, 20))
+    with plan.record(st):
+        ea.agg_sum(col, st)
+    with plan.record(st):
+        with pytest.raises(ea.MsError) as e:
+            ea.release_memory()
+        total = ea.agg_sum(col, st)
+    assert e.value.code == MS_ERR_INVALID
+    plan.launch(st)
+    assert int(total.values(st)[0]) == int(col.values().sum(dtype=np.uint64))
+    del total
+    plan.free()
+
+
+@pytest.mark.parametrize("make", [lambda n: ea.DeviceU64(n), lambda n: hip.DeviceArray(n, np.uint64)])
+def test_failed_device_array(make):
+    x = datagen.uniform_bits(9, 1 << 20, 20)
+    keep = ea.upload_values(x[:10])
+    ea.upload_values(x)
+    kept = used_by_pool()
+    with pytest.raises(RuntimeError):
+        make(1 << 43)
     assert last_error() == 0 and used_by_pool() <= kept - x.nbytes
     assert np.array_equal(keep.values(), x[:10])
