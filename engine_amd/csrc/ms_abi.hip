@@ -395,6 +395,12 @@ struct col_caps {
 static std::mutex g_cols_mu;
 static std::unordered_set<const ms_col *> g_cols;
 
+static bool no_columns()
+{
+    std::lock_guard<std::mutex> lk(g_cols_mu);
+    return g_cols.empty();
+}
+
 // One allocation: [meta 256 B][index][refs][view table][image]
 // A new column; its meta is cleared on the device unless the caller's
 // first kernel writes all of it (clear_meta false).
@@ -784,12 +790,12 @@ extern "C" int ms_col_free(ms_col *c)
     }
     if (c->arena) {
         // arena columns die with their plan
-    } else if (g_rec && g_rec->recording && g_rec->mode == 1) {
+    } else if (plan_capturing()) {
         g_rec->deferred.push_back((void *)c->meta);   // a free now would be captured into the graph
     } else {
         free_ordered((void *)c->meta, c->stream);
-        if (last) cache().drop();
     }
+    if (last && !plan_capturing()) cache().drop();
     delete c->bwi;
     delete c;
     return MS_OK;
@@ -991,6 +997,7 @@ extern "C" int ms_plan_end(ms_plan *p, void *stream)
     hipError_t e = hipStreamEndCapture(p->stream, &p->graph);
     for (void *q : p->deferred) free_ordered(q, p->stream);
     p->deferred.clear();
+    if (no_columns()) cache().drop();
     if (e != hipSuccess) return ms_fail(MS_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
     MS_HIP(hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0));
     return MS_OK;

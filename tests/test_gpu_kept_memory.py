@@ -3,6 +3,7 @@ one call's output to another's scratch, columns read on a created stream
 before they are freed, frees from several threads, and frees while a plan
 captures leave every result as it was."""
 import ctypes
+import gc
 import threading
 
 import numpy as np
@@ -162,3 +163,24 @@ def test_failed_device_array(make):
         make(1 << 43)
     assert last_error() == 0 and used_by_pool() <= kept - x.nbytes
     assert np.array_equal(keep.values(), x[:10])
+
+
+def test_nothing_is_kept_without_columns():
+    """The last column's free gives everything back, also if that column is a
+    plan's."""
+    gc.collect()
+    x = datagen.uniform_bits(9, 1 << 20, 20)
+    keep = ea.upload_values(x[:10])
+    ea.release_memory()
+    before = used_by_pool()
+    st, plan = hip.Stream(), ea.Plan()
+    with plan.record(st):
+        ea.agg_sum(keep, st)
+    with plan.record(st):
+        total = ea.agg_sum(keep, st)
+    ea.upload_values(x)
+    del keep
+    assert used_by_pool() >= before + x.nbytes - 8192
+    del total                                 # the last column
+    assert used_by_pool() < before
+    plan.free()
