@@ -168,9 +168,25 @@ hipError_t device_malloc_async(void **p, size_t bytes, hipStream_t s)
 }
 
 // Frees memory of dev_alloc (or of a created stream) in order on s.
-static void free_ordered(void *p, hipStream_t s)
+static void free_ordered(void *p, hipStream_t s, bool keep = true)
 {
-    if (!cache().put(p)) (void)hipFreeAsync(p, s);
+    if (!cache().put(p, keep)) (void)hipFreeAsync(p, s);
+}
+
+bool unordered_stream(hipStream_t s)
+{
+    if (!s) return false;
+    if (plan_capturing()) return true;
+    unsigned flags = 0;
+    if (hipStreamGetFlags(s, &flags) == hipSuccess) return flags & hipStreamNonBlocking;
+    (void)hipGetLastError();
+    return true;
+}
+
+void col_read(const ms_col *c, hipStream_t s)
+{
+    if (!s || c->stream || c->arena || __atomic_load_n(&c->unordered, __ATOMIC_RELAXED)) return;
+    if (unordered_stream(s)) __atomic_store_n(&c->unordered, true, __ATOMIC_RELAXED);
 }
 
 void *dev_alloc(size_t bytes, hipStream_t s)
@@ -793,7 +809,7 @@ extern "C" int ms_col_free(ms_col *c)
     } else if (plan_capturing()) {
         g_rec->deferred.push_back((void *)c->meta);   // a free now would be captured into the graph
     } else {
-        free_ordered((void *)c->meta, c->stream);
+        free_ordered((void *)c->meta, c->stream, !c->unordered);
     }
     if (last && !plan_capturing()) cache().drop();
     delete c->bwi;
@@ -1212,6 +1228,7 @@ extern "C" int ms_morph(ms_col **out, const ms_format_desc *dst, const ms_col *i
     MS_TRY(ms_need_init());
     if (!out || !in) return ms_fail(MS_ERR_INVALID, "null argument");
     if (!valid_format(dst)) return ms_fail(MS_ERR_INVALID, "invalid destination format");
+    col_read(in, S(stream));
     temps sc(S(stream));
     const uint64_t nb = in->count_bound;
     if (memcmp(dst, &in->f, sizeof *dst) == 0 || (dst->kind == MS_UNCOMPR && in->f.kind == MS_UNCOMPR)) {
@@ -1271,6 +1288,7 @@ extern "C" int ms_morph_blockwise(ms_col **out, const ms_format_desc *dst, const
     if (!out || !in || (!codes && ncodes)) return ms_fail(MS_ERR_INVALID, "null argument");
     if (!valid_format(dst) || dst->kind != MS_BLOCKWISE_INDIVIDUAL)
         return ms_fail(MS_ERR_INVALID, "destination is not a blockwise_individual_f");
+    col_read(in, S(stream));
     uint64_t n;
     MS_TRY(host_count(in, stream, &n));
     if (ncodes != n / dst->block)
@@ -1303,6 +1321,7 @@ static int select_pred(ms_col **out, const ms_pred &p, const ms_format_desc *out
     MS_TRY(ms_need_init());
     if (!out || !in || lanes == 0 || lanes > 64) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
+    col_read(in, S(stream));
     temps sc(S(stream));
     const uint64_t nb = in->count_bound;
     uint64_t *d = (uint64_t *)sc.get(64);
@@ -1375,6 +1394,7 @@ extern "C" int ms_select_sum(uint64_t *d_result, uint32_t cmp, uint64_t val, con
 {
     MS_TRY(ms_need_init());
     if (!d_result || !in || cmp > MS_CMP_GE) return ms_fail(MS_ERR_INVALID, "bad argument");
+    col_read(in, S(stream));
     return launch_select_sum(in, make_pred(cmp, val), d_result, false, S(stream));
 }
 
@@ -1382,6 +1402,7 @@ extern "C" int ms_select_sum_noalloc(uint64_t *d_result, uint32_t cmp, uint64_t 
 {
     MS_TRY(ms_need_init());
     if (!d_result || !in || cmp > MS_CMP_GE) return ms_fail(MS_ERR_INVALID, "bad argument");
+    col_read(in, S(stream));
     int dev = -1;
     MS_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEVICES || !g_scratch_ptr[dev])
@@ -1397,6 +1418,8 @@ extern "C" int ms_project(ms_col **out, const ms_format_desc *out_f, const ms_co
     MS_TRY(ms_need_init());
     if (!out || !data || !pos || lanes == 0 || lanes > 64) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
+    col_read(data, S(stream));
+    col_read(pos, S(stream));
     temps sc(S(stream));
     const uint64_t np = pos->count_bound;
     const uint64_t *pv, *d_np;
@@ -1453,6 +1476,7 @@ extern "C" int ms_agg_sum(ms_col **out, const ms_col *in, void *stream)
 {
     MS_TRY(ms_need_init());
     if (!out || !in) return ms_fail(MS_ERR_INVALID, "bad argument");
+    col_read(in, S(stream));
     ms_col *c;
     MS_TRY(new_col(uncompr_desc(), 1, 64, S(stream), &c, nullptr, false));
     ms_pred all = make_pred(MS_CMP_GE, 0);
@@ -1471,6 +1495,8 @@ extern "C" int ms_group(ms_col **out_gr, ms_col **out_ext, const ms_format_desc 
     if (!valid_format(gr_f) || !wit_ok(gr_f) || !valid_format(ext_f) || !wit_ok(ext_f))
         return ms_fail(MS_ERR_INVALID, "invalid output format");
     if (plan_capturing()) return ms_fail(MS_ERR_INVALID, "group synchronises: not in a plan");
+    col_read(in_data, S(stream));
+    if (in_gr) col_read(in_gr, S(stream));
     uint64_t n, ng;
     MS_TRY(host_count(in_data, stream, &n));
     if (in_gr) {
@@ -1505,6 +1531,8 @@ extern "C" int ms_join(ms_col **out_l, ms_col **out_r, const ms_format_desc *l_f
     if (!valid_format(l_f) || !wit_ok(l_f) || !valid_format(r_f) || !wit_ok(r_f))
         return ms_fail(MS_ERR_INVALID, "invalid output format");
     if (plan_capturing()) return ms_fail(MS_ERR_INVALID, "join synchronises: not in a plan");
+    col_read(l, S(stream));
+    col_read(r, S(stream));
     uint64_t na, nb;
     MS_TRY(host_count(l, stream, &na));
     MS_TRY(host_count(r, stream, &nb));
@@ -1537,6 +1565,8 @@ extern "C" int ms_semi_join(ms_col **out, const ms_format_desc *out_f, const ms_
     if (!out || !l || !r) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
     if (plan_capturing()) return ms_fail(MS_ERR_INVALID, "join synchronises: not in a plan");
+    col_read(l, S(stream));
+    col_read(r, S(stream));
     uint64_t na, nb;
     MS_TRY(host_count(l, stream, &na));
     MS_TRY(host_count(r, stream, &nb));
@@ -1560,6 +1590,8 @@ extern "C" int ms_intersect_sorted(ms_col **out, const ms_format_desc *out_f, co
     MS_TRY(ms_need_init());
     if (!out || !l || !r) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
+    col_read(l, S(stream));
+    col_read(r, S(stream));
     temps sc(S(stream));
     const uint64_t *a, *b, *d_na, *d_nb;
     MS_TRY(values_of(l, sc, &a, &d_na));
@@ -1579,6 +1611,8 @@ extern "C" int ms_merge_sorted(ms_col **out, const ms_format_desc *out_f, const 
     MS_TRY(ms_need_init());
     if (!out || !l || !r) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
+    col_read(l, S(stream));
+    col_read(r, S(stream));
     temps sc(S(stream));
     const uint64_t *a, *b, *d_na, *d_nb;
     MS_TRY(values_of(l, sc, &a, &d_na));
@@ -1612,6 +1646,8 @@ extern "C" int ms_calc_binary(ms_col **out, uint32_t op, const ms_format_desc *o
     MS_TRY(ms_need_init());
     if (!out || !l || !r || op > MS_OP_XOR) return ms_fail(MS_ERR_INVALID, "bad argument");
     if (!valid_format(out_f) || !wit_ok(out_f)) return ms_fail(MS_ERR_INVALID, "invalid output format");
+    col_read(l, S(stream));
+    col_read(r, S(stream));
     if (!plan_capturing()) {
         // eagerly the mismatch is an error of this call, as in the reference
         ms_col_meta ml, mr;

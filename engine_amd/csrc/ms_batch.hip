@@ -565,6 +565,8 @@ static int launch(ms_batch *b, uint64_t *d_results, hipStream_t s)
 {
     const uint64_t nE = b->E.size();
     if (nE == 0) return MS_OK;
+    if (unordered_stream(s))
+        for (const ms_col *c : b->cols) col_read(c, s);
     const bool u2 = b->cfg.unroll == 2;
     auto kern = b->cfg.waves_per_simd == 8 ? (u2 ? k_batch_select_sum_w8_u2 : k_batch_select_sum_w8)
               : b->cfg.waves_per_simd == 6 ? k_batch_select_sum_w6
@@ -761,6 +763,8 @@ extern "C" int ms_batch_view_times(ms_batch *b, uint64_t *d_results, uint32_t re
     MS_HIP(hipGetDevice(&dev));
     MS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
     if (khz <= 0) return ms_fail(MS_ERR_HIP, "no wall clock rate");
+    if (unordered_stream(s))
+        for (const ms_col *c : b->cols) col_read(c, s);
     unsigned long long *ticks = nullptr;
     MS_HIP(device_malloc_async((void **)&ticks, std::max<uint64_t>(b->ntags, 1) * 8, s));
     int rc = launch_fill_u64((uint64_t *)ticks, std::max<uint64_t>(b->ntags, 1), 0, s);

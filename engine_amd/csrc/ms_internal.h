@@ -257,4 +257,5 @@ struct ms_col {
     bool prepared;
     ms_bwi *bwi;             // blockwise_individual_f: the views (host)
     ms_dev_meta *vmeta;      // blockwise_individual_f: meta of every view, then of the 3 groups
+    mutable bool unordered;  // a stream that the null stream does not wait for has read it (ms::col_read)
 };

@@ -6,7 +6,8 @@
 // kernels) that was 0.8 to 12 ms, growing with the memory the process holds.
 // A block freed on the null stream is handed to a later call on the null
 // stream without waiting: the stream orders its uses, and unlike a created
-// stream it is never destroyed and never captured; other streams keep
+// stream it is never destroyed and never captured; created streams, which it
+// waits for, may read a block until then; other streams keep
 // using hipMallocAsync.  At most a sixteenth of a device's memory is kept (the
 // least recently freed blocks go first).
 //
@@ -134,9 +135,9 @@ public:
         return hold(k);
     }
 
-    // Takes back memory of get(), whatever device is current.  false: not a
-    // block of this object.
-    bool put(void *p)
+    // Takes back memory of get(), whatever device is current; `keep` false:
+    // to the pool, not for a later call.  false: not a block of this object.
+    bool put(void *p, bool keep = true)
     {
         std::lock_guard<std::mutex> lk(mu);
         auto l = live.find(p);
@@ -149,7 +150,7 @@ public:
             const size_t total = Api::total(k.dev);
             d.limit = total ? total / 16 : 1u << 30;
         }
-        if (k.bytes > d.limit) {
+        if (!keep || k.bytes > d.limit) {
             Api::free(k.dev, p);
             return true;
         }

@@ -49,6 +49,13 @@ hipError_t device_malloc_async(void **p, size_t bytes, hipStream_t s);
 // device holds at once, queried once per kernel.
 uint32_t resident_grid(const void *kernel, uint32_t wg);
 
+// Notes that a call on s reads c.  The null stream waits for the created
+// streams, so a block it freed may serve its next call while they still read
+// it, but not for non-blocking ones, and a plan may be launched on any: a
+// column that one of these read is freed to the pool instead of kept.
+bool unordered_stream(hipStream_t s);
+void col_read(const ms_col *c, hipStream_t s);
+
 // Bytes of a column's meta at the start of its allocation; index,
 // references and view table, where it has them, and its image follow.
 constexpr uint64_t COL_META_BYTES = 256;

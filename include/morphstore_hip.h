@@ -247,7 +247,10 @@ int ms_col_load(ms_col **out, const ms_format_desc *f, const char *path, void *s
 
 /* Releases the column, stream ordered on the stream it was created on:
  * that stream must still exist (destroy a stream only after freeing the
- * columns created on it; the null stream always exists). */
+ * columns created on it; the null stream always exists).  Work of the
+ * caller's own that reads ms_col_device_data on a stream which that stream
+ * does not wait for (another created one; a non-blocking one for a column of
+ * the null stream) must be done, or waited for by that stream, before. */
 int ms_col_free(ms_col *c);
 
 /* ------------------------------------------------------------------ */

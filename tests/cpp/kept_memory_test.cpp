@@ -93,6 +93,7 @@ static void reuse(kept &k)
     CHECK(c != a && c != b);                  // never to two calls
     CHECK(k.put(b) && k.get(MiB) != b);       // far too large
     CHECK(fake::frees == 0);
+    CHECK(k.put(c, false) && !fake::held.count(c) && fake::frees == 1);   // not to be kept
 }
 
 // A sixteenth of the device is kept; the least recently freed goes first.

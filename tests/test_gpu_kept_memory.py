@@ -1,7 +1,9 @@
 """Memory of the null stream is kept for its next calls: blocks that go from
 one call's output to another's scratch, columns read on a created stream
 before they are freed, frees from several threads, and frees while a plan
-captures leave every result as it was."""
+captures leave every result as it was.  What is kept goes back when an
+allocation fails, with the last column and on request, and is not what a
+non-blocking stream or a plan reads."""
 import ctypes
 import gc
 import threading
@@ -11,8 +13,8 @@ import pytest
 
 import engine_amd as ea
 from engine_amd import datagen, hip
-from engine_amd.formats import (MS_CMP_LT, MS_ERR_INVALID, MS_ERR_NOMEM, default_delta_dynamic_vbp_f, dynamic_vbp_f,
-                                rle_f, uncompr_f)
+from engine_amd.formats import (MS_CMP_GE, MS_CMP_LT, MS_ERR_INVALID, MS_ERR_NOMEM, MS_OP_ADD, blockwise_individual_f,
+                                default_delta_dynamic_vbp_f, dynamic_vbp_f, rle_f, uncompr_f)
 
 pytestmark = pytest.mark.gpu
 
@@ -184,3 +186,92 @@ def test_nothing_is_kept_without_columns():
     del total                                 # the last column
     assert used_by_pool() < before
     plan.free()
+
+
+class NonBlocking:
+    """A created stream that the null stream does not wait for."""
+
+    def __init__(self):
+        self._as_parameter_ = ctypes.c_void_p()
+        assert hip.hip().hipStreamCreateWithFlags(ctypes.byref(self._as_parameter_), 1) == 0
+
+    def synchronize(self):
+        assert hip.hip().hipStreamSynchronize(self._as_parameter_) == 0
+
+    def destroy(self):
+        assert hip.hip().hipStreamDestroy(self._as_parameter_) == 0
+
+
+D = dynamic_vbp_f(512, 2048, 8)
+
+
+def batch_run(col, pos, st, res):
+    b = ea.Batch()
+    b.enqueue(col, MS_CMP_LT, 9)
+    b.run(res, st)
+    return b
+
+
+READS = {
+    "select_sum": lambda col, pos, st, res: ea.select_sum(MS_CMP_LT, 9, col, res, st),
+    "select_sum_noalloc": lambda col, pos, st, res: ea.select_sum_noalloc(MS_CMP_LT, 9, col, res, st),
+    "morph": lambda col, pos, st, res: ea.morph(D, col, st),
+    "morph_blockwise": lambda col, pos, st, res: ea.morph_blockwise(blockwise_individual_f(1024), col,
+                                                                    np.full(1024, 65, np.uint8), st),
+    "select": lambda col, pos, st, res: ea.select(MS_CMP_LT, 9, uncompr_f(), col, 8, st),
+    "between": lambda col, pos, st, res: ea.between(MS_CMP_GE, 2, MS_CMP_LT, 9, uncompr_f(), col, 8, st),
+    "project_data": lambda col, pos, st, res: ea.project(uncompr_f(), col, pos, 8, st),
+    "project_pos": lambda col, pos, st, res: ea.project(uncompr_f(), col, col, 8, st),
+    "agg_sum": lambda col, pos, st, res: ea.agg_sum(col, st),
+    "intersect_l": lambda col, pos, st, res: ea.intersect_sorted(uncompr_f(), col, pos, st),
+    "intersect_r": lambda col, pos, st, res: ea.intersect_sorted(uncompr_f(), pos, col, st),
+    "merge_l": lambda col, pos, st, res: ea.merge_sorted(uncompr_f(), col, pos, st),
+    "merge_r": lambda col, pos, st, res: ea.merge_sorted(uncompr_f(), pos, col, st),
+    "calc": lambda col, pos, st, res: ea.calc_binary(MS_OP_ADD, uncompr_f(), col, col, st),
+    "group": lambda col, pos, st, res: ea.group(uncompr_f(), uncompr_f(), col, None, st),
+    "group_of": lambda col, pos, st, res: ea.group(uncompr_f(), uncompr_f(), col, col, st),
+    "join": lambda col, pos, st, res: ea.join(uncompr_f(), uncompr_f(), pos, col, st),
+    "semi_join": lambda col, pos, st, res: ea.semi_join(uncompr_f(), pos, col, st),
+    "batch": batch_run,
+}
+
+
+@pytest.mark.parametrize("op", READS)
+def test_columns_read_on_a_non_blocking_stream(op):
+    """They go to the pool: the null stream's next call does not wait for
+    such a stream.  Read on a blocking one they are kept."""
+    for st, kept in ((NonBlocking(), False), (hip.Stream(), True)):
+        res = ea.DeviceU64()
+        pos = ea.upload_values(np.arange(40, dtype=np.uint64))
+        ea.release_memory()
+        before = used_by_pool()
+        col = ea.upload_values(np.arange(1 << 20, dtype=np.uint64))
+        hip.synchronize()
+        out = READS[op](col, pos, st, res)
+        st.synchronize()
+        del out
+        del col
+        assert (used_by_pool() >= before + (8 << 20)) == kept
+        if not kept:
+            st.destroy()
+
+
+def test_columns_read_by_a_plan():
+    """A plan may be launched on any stream."""
+    st, plan = hip.Stream(), ea.Plan()
+    keep = ea.upload_values(np.arange(40, dtype=np.uint64))
+    ea.release_memory()
+    before = used_by_pool()
+    col = ea.upload_values(np.arange(1 << 20, dtype=np.uint64))
+    hip.synchronize()
+    with plan.record(st):
+        ea.agg_sum(col, st)
+    with plan.record(st):
+        total = ea.agg_sum(col, st)
+    plan.launch(st)
+    assert int(total.values(st)[0]) == (1 << 19) * ((1 << 20) - 1)
+    del total
+    plan.free()
+    del col
+    assert used_by_pool() < before + (8 << 20)
+    assert len(keep.values()) == 40
