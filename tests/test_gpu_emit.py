@@ -58,3 +58,11 @@ def test_write_iterator_emission(oracle, f):
         o = oracle.calc_binary(MS_OP_XOR, f, oracle.morph(ea.FormatDesc(0), v), oracle.morph(ea.FormatDesc(0), z))
         same(g, o)
 
+
+@pytest.mark.parametrize("f", [FORMATS[0], FORMATS[4], FORMATS[8]], ids=repr)
+def test_column_emission_many_tiles(oracle, f):
+    # 4096 tiles, several per resident workgroup: its words, references and
+    # deferred tile are reused; blocks of every width, so that tiles packed in
+    # LDS and tiles with blocks read again follow each other
+    v = values("wide", 1 << 26)
+    same(ea.morph(f, ea.upload_values(v)), oracle.morph(f, v))

@@ -41,3 +41,14 @@ def test_merge_one_value_and_disjoint(na, nb):
         a, b = a.astype(np.uint64), b.astype(np.uint64)
         got = ea.merge_sorted(uncompr_f(), ea.upload_values(a), ea.upload_values(b)).values()
         assert np.array_equal(got, union(a, b))
+
+
+def test_merge_many_tiles():
+    # 4800 tiles, several per resident workgroup: its staged values are reused
+    r = datagen.splitmix64(3, 2 * 20_000_000)
+    gaps = (r >> np.uint64(62)) + np.uint64(1)
+    a, b = np.cumsum(gaps[:20_000_000], dtype=np.uint64), np.cumsum(gaps[20_000_000:], dtype=np.uint64)
+    either = np.zeros(int(max(a[-1], b[-1])) + 1, bool)
+    either[a] = either[b] = True
+    got = ea.merge_sorted(uncompr_f(), ea.upload_values(a), ea.upload_values(b)).values()
+    assert np.array_equal(got, np.flatnonzero(either).astype(np.uint64))

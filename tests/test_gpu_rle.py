@@ -38,3 +38,15 @@ def test_rle_both_ways(oracle, lens):
         assert meta == o.meta(), n
         assert img.tobytes() == o.image().tobytes(), n
         assert np.array_equal(ea.morph(uncompr_f(), g).values(), v), n
+
+
+@pytest.mark.parametrize("lens", [[1, 2], [5] * 20_000 + [9] * 20_000], ids=lambda x: str(x[:2]))
+def test_rle_both_ways_many_tiles(oracle, lens):
+    # 4096 tiles, several per resident workgroup: its kept heads are reused;
+    # every wave beyond its 256 kept heads, and waves on either side of that
+    v = runs_of(lens, 1 << 26)
+    g = ea.morph(rle_f(), ea.upload_values(v))
+    o = oracle.morph(rle_f(), v)
+    img, meta = g.image()
+    assert meta == o.meta() and np.array_equal(img, o.image())
+    assert np.array_equal(ea.morph(uncompr_f(), g).values(), v)

@@ -48,3 +48,16 @@ def test_select_positions_long(n):
         col = ea.morph(f, ea.upload_values(x)) if f.kind else ea.upload_values(x)
         for cmp, val in [(MS_CMP_LT, 1 << 11), (MS_CMP_EQ, 77)]:
             assert np.array_equal(ea.select(cmp, val, uncompr_f(), col, 8).values(), rm.select_positions(x, cmp, val))
+
+
+@pytest.mark.parametrize("f", [static_vbp_f(12, 1), dynamic_vbp_f(512, 2048, 8), uncompr_f()], ids=repr)
+def test_select_positions_many_tiles(f):
+    # 4097 tiles of 32768 rows, several per resident workgroup: its row words
+    # and ticket are reused from turn to turn
+    n = (1 << 27) + 77
+    x = (np.arange(n, dtype=np.uint64) * np.uint64(0x9E3779B97F4A7C15)) >> np.uint64(52)
+    col = ea.upload_values(x)
+    if f.kind:
+        col = ea.morph(f, col)
+    for cmp, val in [(MS_CMP_LT, 1 << 11), (MS_CMP_EQ, 77)]:
+        assert np.array_equal(ea.select(cmp, val, uncompr_f(), col, 8).values(), rm.select_positions(x, cmp, val))
