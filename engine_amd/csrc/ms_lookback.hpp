@@ -4,9 +4,20 @@
 // tiles in ticket order and publishes one 64-bit word per tile: first the
 // tile's own total, then (once known) the total of all tiles up to it.  A
 // tile's offset is found by one wave reading 64 predecessors' words at a
-// time.  Progress: a tile's ticket is only handed out after every earlier
-// ticket, so each word that is waited for belongs to a workgroup that
-// already runs, and a tile publishes its total before it waits.
+// time.  Progress: tickets are handed out in order to workgroups that already
+// run.  A kernel that looks back for the tile it holds (k_merge, k_rle_starts)
+// publishes that tile's total first.  One that looks back a tile late
+// (k_emit_onepass, k_rle_onepass, k_select_onepass) holds up to three tickets:
+// the tile that waits for its offset, a later one whose total it publishes
+// before that wait, and the next one, whose total comes after it.  In both a
+// workgroup only ever waits for words of tiles below one that it has published
+// itself, and its tickets ascend; so the owner of the lowest unpublished tile
+// waits, if at all, for published words only, and goes on to publish.  Totals
+// are enough for that: a wait ends with the words of all tiles below, prefix
+// or not.  The page starts of k_emit_onepass are words of the same kind, stored
+// by a page's first tile at its own look-back and waited for by the page's
+// later tiles after theirs: the lowest tile whose look-back is not done waits
+// for no page start that is not stored.
 // The words and the ticket counter are cleared before the launch.
 #pragma once
 
