@@ -1521,9 +1521,19 @@ int launch_select_positions(const ms_col *in, const ms_pred &p, uint64_t *d_pos,
     ms_colv v;
     MS_TRY(colv_of(in, v));
     // few units per wave while that leaves CUs without a tile, many for few
-    // tickets (2^18 rows: 8.1 / 9.3 / 13.4 us with 1 / 2 / 4 units, 2^24
-    // rows: 47 / 39 / 34 us)
-    const uint32_t per_wave = nb <= 1ull << 21 ? 1 : nb <= 1ull << 23 ? 2 : SEL_UNITS;
+    // tickets.  Calls one after the other, 1 / 2 / 4 units, us, half of the
+    // rows selected:
+    //   rows     static_vbp_f<12, 1>   dynamic_vbp_f       uncompr_f
+    //   2^18     11.5 / 12.3 / 16.9    10.3 / 11.9 / 15.6  10.5 / 12.3 / 15.8
+    //   2^20     12.2 / 13.3 / 17.6    12.3 / 12.6 / 15.5  12.4 / 13.2 / 16.5
+    //   2^20.5   15.5 / 14.3 / 17.8    15.4 / 12.9 / 16.0  15.3 / 13.9 / 17.9
+    //   2^21     18.1 / 14.6 / 18.2    18.5 / 14.6 / 16.7  18.6 / 15.2 / 19.0
+    //   2^23     32.6 / 27.2 / 30.5    33.6 / 27.6 / 30.4  34.0 / 29.9 / 37.2
+    //   2^23.5   39.8 / 32.6 / 32.3    41.1 / 33.1 / 32.2  42.7 / 39.1 / 39.2
+    //   2^24     50.3 / 40.1 / 35.8    51.9 / 40.2 / 35.0  54.4 / 48.9 / 44.1
+    // (4 are 10% better around 2^22 from the packed sources: one round of
+    // tiles per resident workgroup.)
+    const uint32_t per_wave = nb <= 1ull << 20 ? 1 : nb <= 1ull << 23 ? 2 : SEL_UNITS;
     const uint64_t tiles = nb / (512ull * SEL_WAVES * per_wave) + 1;
     uint64_t *state = (uint64_t *)sc.get((1 + tiles) * 8);
     if (!state) return ms_fail(MS_ERR_NOMEM, "select scratch");
