@@ -234,15 +234,17 @@ __global__ __launch_bounds__(WG) void k_select_sum_rle(ms_colv c, ms_pred p, ss_
 // running sums of the S lanes at the tile's start (its "carries"), so every
 // tile decodes independently: a workgroup (4 waves x 512 values) scans its
 // tile locally and adds the carries.  SRC 0 decodes 8-lane indexed blocks,
-// SRC 1 reads deltas already decoded into `arr`.
+// SRC 1 reads deltas already decoded into `arr`, whose n need not end with a
+// unit of 512 (blocks of fewer values).
 // ------------------------------------------------------------------
 static constexpr uint64_t DELTA_TILE = MS_DELTA_TILE;
 static_assert(MS_DELTA_TILE == WAVES * 512, "a delta tile is one workgroup's 4 units");
 
 template <int SRC>
 // e_v: unit u's index entry (SRC 0), loaded by the caller.
-__device__ __forceinline__ void delta_load(const ms_colv &c, const uint64_t *arr, uint64_t u, uint64_t nunits,
-                                           uint32_t S, uint32_t j, uint32_t gl, uint64_t e_v, uint64_t (&d)[8])
+__device__ __forceinline__ void delta_load(const ms_colv &c, const uint64_t *arr, uint64_t n, uint64_t u,
+                                           uint64_t nunits, uint32_t S, uint32_t j, uint32_t gl, uint64_t e_v,
+                                           uint64_t (&d)[8])
 {
     if (u >= nunits) {
 #pragma unroll
@@ -255,8 +257,14 @@ __device__ __forceinline__ void delta_load(const ms_colv &c, const uint64_t *arr
         dec_dispatch((uint32_t)(e & 0xff), (const uint64_t *)(c.data + (e >> 8)), 8, j, sub * 8 + gl, d);
     } else {
         const uint64_t *a = arr + u * 512;
+        if ((u + 1) * 512 <= n) {
 #pragma unroll
-        for (int m = 0; m < 8; m++) d[m] = a[S * (8 * gl + m) + j];
+            for (int m = 0; m < 8; m++) d[m] = a[S * (8 * gl + m) + j];
+        } else {
+            const uint32_t left = (uint32_t)(n - u * 512);
+#pragma unroll
+            for (int m = 0; m < 8; m++) d[m] = S * (8 * gl + m) + j < left ? a[S * (8 * gl + m) + j] : 0;
+        }
     }
 }
 
@@ -295,7 +303,7 @@ __global__ __launch_bounds__(WG) void k_delta_tiles(ms_colv c, const uint64_t *a
     __shared__ uint64_t s_wtot[WAVES][8];
     const ms_parts pt = parts_of(c);
     const uint32_t S = c.g.dstep;
-    const uint64_t nunits = pt.n_compr >> 9;
+    const uint64_t nunits = (pt.n_compr + 511) >> 9;   // SRC 0: all of them full
     const uint64_t ntiles = (nunits + WAVES - 1) / WAVES;
     const uint32_t wv = wave_index();
     const uint32_t t = threadIdx.x & 63;
@@ -311,19 +319,26 @@ __global__ __launch_bounds__(WG) void k_delta_tiles(ms_colv c, const uint64_t *a
         const uint64_t un = (tile + gridDim.x) * WAVES + wv;
         if (SRC == 0) e_n = un < nunits ? gload(c.index + (un >> c.g.lg_spb)) : 0ull;
         uint64_t d[8];
-        delta_load<SRC>(c, arr, u, nunits, S, j, gl, e_v, d);
+        delta_load<SRC>(c, arr, pt.n_compr, u, nunits, S, j, gl, e_v, d);
         uint64_t tile_tot;
         const uint64_t base = carry + delta_tile_scan(d, S, j, t, wv, s_wtot, tile_tot);
         if (u < nunits) {
+            const uint32_t left = SRC == 0 || (u + 1) * 512 <= pt.n_compr ? 512u : (uint32_t)(pt.n_compr - u * 512);
             if (MODE == 0) {
                 uint64_t *o = out + u * 512;
+                if (left == 512) {
 #pragma unroll
-                for (int m = 0; m < 8; m++) o[S * (8 * gl + m) + j] = base + d[m];
+                    for (int m = 0; m < 8; m++) o[S * (8 * gl + m) + j] = base + d[m];
+                } else {
+#pragma unroll
+                    for (int m = 0; m < 8; m++)
+                        if (S * (8 * gl + m) + j < left) o[S * (8 * gl + m) + j] = base + d[m];
+                }
             } else {
 #pragma unroll
                 for (int m = 0; m < 8; m++) {
                     const uint64_t x = base + d[m];
-                    acc += pred_eval(p, x) ? x : 0;
+                    acc += S * (8 * gl + m) + j < left && pred_eval(p, x) ? x : 0;
                 }
             }
         }
@@ -361,7 +376,7 @@ __global__ __launch_bounds__(WG) void k_delta_tile_sums(ms_colv c, const uint64_
     __shared__ uint64_t s_wtot[WAVES][8];
     const ms_parts pt = parts_of(c);
     const uint32_t S = c.g.dstep;
-    const uint64_t nunits = pt.n_compr >> 9;
+    const uint64_t nunits = (pt.n_compr + 511) >> 9;
     const uint32_t wv = wave_index();
     const uint32_t t = threadIdx.x & 63;
     const uint32_t j = t & (S - 1), gl = t >> c.g.lg_dstep;
@@ -369,7 +384,7 @@ __global__ __launch_bounds__(WG) void k_delta_tile_sums(ms_colv c, const uint64_
         const uint64_t u = tile * WAVES + wv;
         const uint64_t e_v = SRC == 0 && u < nunits ? gload(c.index + (u >> c.g.lg_spb)) : 0ull;
         uint64_t d[8];
-        delta_load<SRC>(c, arr, u, nunits, S, j, gl, e_v, d);
+        delta_load<SRC>(c, arr, pt.n_compr, u, nunits, S, j, gl, e_v, d);
         uint64_t tile_tot;
         (void)delta_tile_scan(d, S, j, t, wv, s_wtot, tile_tot);
         if (threadIdx.x < S) sums[(uint64_t)threadIdx.x * ntb + tile] = tile_tot;
