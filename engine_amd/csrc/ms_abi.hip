@@ -1341,7 +1341,7 @@ static int select_pred(ms_col **out, const ms_pred &p, const ms_format_desc *out
     uint64_t *pos = (uint64_t *)sc.get(nb * 8 + 64);
     if (!pos) return ms_fail(MS_ERR_NOMEM, "select scratch");
     if (select_flags_ok(in) && emit_flags_ok(*out_f)) {
-        // positions go from the count pass's ballots straight into the
+        // positions go from the count pass's flag bytes straight into the
         // output format; pos only receives the few read by rank
         sel_flags sf;
         MS_TRY(launch_select_flags(in, p, sf, sc));

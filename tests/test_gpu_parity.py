@@ -124,7 +124,7 @@ def test_select_byte_identical(oracle, lanes, out_f, in_f):
 
 
 # select from dynamic_vbp / for_f inputs into the block formats packs its
-# output straight from the count pass's ballots: densities from a handful
+# output straight from the count pass's flags: densities from a handful
 # of rows to all of them (units walked past empty, lanes full), delta steps
 # equal to and below the lane count, and inner blocks of 512 to 2048
 @pytest.mark.parametrize("out_f", [default_delta_dynamic_vbp_f(8), delta_f(1024, 4, dynamic_vbp_f(512, 64, 4)),
@@ -146,7 +146,7 @@ def test_select_positions_from_ballots(oracle, out_f, in_f):
 
 @pytest.mark.parametrize("in_f", [dynamic_vbp_f(512, 2048, 8), default_for_dynamic_vbp_f(8)], ids=repr)
 def test_select_positions_from_ballots_small_and_ragged(oracle, in_f):
-    """The ballot-fed emit at the edges: empty and one-value inputs, counts
+    """The flag-fed emit at the edges: empty and one-value inputs, counts
     around a unit, a delta tile and a write-iterator flush, with and
     without a scalar remainder."""
     for n in (0, 1, 5, 511, 512, 513, 1023, 2049, 4095, 4097):
