@@ -558,25 +558,6 @@ constexpr uint32_t RLE_XT = 2048;       // values per output tile
 constexpr uint32_t RLE_SCH = 64;        // chunks per tile of k_rle_starts
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-// Inclusive sum over the wave (DPP).
-__device__ __forceinline__ uint64_t dpp_scan_u64(uint64_t x)
-{
-#define MS_DPP_ADD(ctl, rows)                                                                                     \
-    {                                                                                                             \
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, ctl, rows, 0xf, false);    \
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), ctl, rows, 0xf, false); \
-        x += ((uint64_t)hi << 32) | lo;                                                                           \
-    }
-    MS_DPP_ADD(0x111, 0xf)   // row_shr:1, 2, 4, 8
-    MS_DPP_ADD(0x112, 0xf)
-    MS_DPP_ADD(0x114, 0xf)
-    MS_DPP_ADD(0x118, 0xf)
-    MS_DPP_ADD(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
-    MS_DPP_ADD(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
-#undef MS_DPP_ADD
-    return x;
-}
-
 // Clears the look-back state and sets the expanded column's meta.
 __global__ __launch_bounds__(WG) void k_rle_begin(const ms_dev_meta *in, uint64_t *state, uint64_t words,
                                                   ms_dev_meta *om)
@@ -690,32 +671,22 @@ __global__ __launch_bounds__(WG) void k_rle_expand(ms_colv c, const uint64_t *cs
                 if (pos >= o0 + size) break;
                 continue;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             const uint32_t p0 = start > o0 ? (uint32_t)(start - o0) : 0u;
             if (in) {
-                const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                const uint32_t k = lanes_below(m);
                 s_val[w][k] = vl.x;
                 atomicOr(&s_bits[w][p0 >> 5], 1u << (p0 & 31));
             }
             // the values this batch writes: [lo, hi) of the tile
             const uint32_t lo = __builtin_amdgcn_readlane(p0, __builtin_ctzll(m));
             const uint32_t hi = pos - o0 < size ? (uint32_t)(pos - o0) : size;
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             const uint32_t bits = s_bits[w][t];
-            uint32_t heads = (uint32_t)__builtin_popcount(bits);
-            const uint32_t own = heads;
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x111, 0xf, 0xf, false);
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x112, 0xf, 0xf, false);
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x114, 0xf, 0xf, false);
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x118, 0xf, 0xf, false);
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x142, 0xa, 0xf, false);
-            heads += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)heads, 0x143, 0xc, 0xf, false);
+            const uint32_t own = (uint32_t)__builtin_popcount(bits);
+            const uint32_t heads = dpp_scan_u32(own, op_add{});
             s_word[w][t] = u32x2{bits, heads - own};
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
             for (uint32_t row = lo / 128; row * 128 < hi; row++) {
                 const uint32_t p = row * 128 + 2 * t;
                 const u32x2 wd = s_word[w][p >> 5];
@@ -736,8 +707,7 @@ __global__ __launch_bounds__(WG) void k_rle_expand(ms_colv c, const uint64_t *cs
                 }
             }
             if (pos >= o0 + size) break;
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            wave_lds_sync();
         }
     }
 }
@@ -1251,18 +1221,6 @@ __device__ __forceinline__ uint32_t flag_finish(const uint8_t *data, const ms_pr
     return mode == SM_OUT ? bits ^ 0xffu : bits;
 }
 
-// Sum over the wave (DPP), uniform.
-__device__ __forceinline__ uint32_t dpp_sum_u32(uint32_t x)
-{
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);
-    return __builtin_amdgcn_readlane(x, 63);
-}
-
 // Decodes and tests every unit once: each thread's flag byte goes to byte t
 // of the unit's flags (64 bytes per 512 values) and its selected count to
 // cnt[u].  As the fused sums do, a wave takes 4 units at a time: each unit's
@@ -1468,8 +1426,7 @@ __global__ __launch_bounds__(SEL_WAVES * 64) void k_select_onepass(ms_colv c, co
                 const uint64_t F = readlane64(mine_w, r);
                 if (F == 0) continue;
                 if (__builtin_amdgcn_inverse_ballot_w64(F))
-                    pos[o + __builtin_amdgcn_mbcnt_hi((uint32_t)(F >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)F, 0))] =
-                        u0 * 512 + 64 * r + t;
+                    pos[o + lanes_below(F)] = u0 * 512 + 64 * r + t;
                 o += (uint32_t)__popcll(F);
             }
             if (ptile == ntiles - 1 && threadIdx.x == 0) {

@@ -180,6 +180,68 @@ __device__ __forceinline__ uint64_t wave_or_u64(uint64_t x)
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
+// Lanes below this one in a mask of lanes.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// Orders a wave's LDS accesses among its lanes (LDS serves one wave in order).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Inclusive scan over the wave by DPP; lanes without a partner combine with 0.
+#define MS_DPP_STEP(ctl, rows) \
+    x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctl, rows, 0xf, false));
+template <class Op>
+__device__ __forceinline__ uint32_t dpp_scan_u32(uint32_t x, const Op &op)
+{
+    MS_DPP_STEP(0x111, 0xf)   // row_shr:1, 2, 4, 8
+    MS_DPP_STEP(0x112, 0xf)
+    MS_DPP_STEP(0x114, 0xf)
+    MS_DPP_STEP(0x118, 0xf)
+    MS_DPP_STEP(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
+    MS_DPP_STEP(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
+    return x;
+}
+#undef MS_DPP_STEP
+
+struct op_add {
+    __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return a + b; }
+};
+struct op_max {
+    __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return b > a ? b : a; }
+};
+
+// Sum and maximum over the wave, uniform.
+__device__ __forceinline__ uint32_t dpp_sum_u32(uint32_t x)
+{
+    return __builtin_amdgcn_readlane(dpp_scan_u32(x, op_add{}), 63);
+}
+__device__ __forceinline__ uint32_t dpp_max_u32(uint32_t x)
+{
+    return __builtin_amdgcn_readlane(dpp_scan_u32(x, op_max{}), 63);
+}
+
+// Inclusive 64-bit sum over the wave.
+__device__ __forceinline__ uint64_t dpp_scan_u64(uint64_t x)
+{
+#define MS_DPP_HALF(y, ctl, rows) (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(y), ctl, rows, 0xf, false)
+#define MS_DPP_ADD(ctl, rows) x += ((uint64_t)MS_DPP_HALF(x >> 32, ctl, rows) << 32) | MS_DPP_HALF(x, ctl, rows);
+    MS_DPP_ADD(0x111, 0xf)
+    MS_DPP_ADD(0x112, 0xf)
+    MS_DPP_ADD(0x114, 0xf)
+    MS_DPP_ADD(0x118, 0xf)
+    MS_DPP_ADD(0x142, 0xa)
+    MS_DPP_ADD(0x143, 0xc)
+#undef MS_DPP_ADD
+#undef MS_DPP_HALF
+    return x;
+}
+
 // Bit m of byte j to bit j of byte m (an 8 x 8 transpose in three swaps of
 // ever larger blocks): a select's flag word to its 64 rows in order.
 __device__ __forceinline__ uint64_t flag_rows(uint64_t x)

@@ -724,31 +724,6 @@ constexpr uint32_t OP_TILE = OP_WAVES * OP_WB;   // blocks per tile
 constexpr uint32_t OP_B = 512, OP_S = 8;
 constexpr uint32_t OP_SLOT = 256;                // LDS words per block: codes of up to 32 bits
 
-// Maximum over the wave (a DPP reduction into lane 63), uniform.
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x)
-{
-#define MS_DPP_MAX(ctl, rows)                                                                              \
-    {                                                                                                      \
-        const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctl, rows, 0xf, false);        \
-        x = y > x ? y : x;                                                                                 \
-    }
-    MS_DPP_MAX(0x111, 0xf)   // row_shr:1, 2, 4, 8: each row's maximum in its last lane
-    MS_DPP_MAX(0x112, 0xf)
-    MS_DPP_MAX(0x114, 0xf)
-    MS_DPP_MAX(0x118, 0xf)
-    MS_DPP_MAX(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
-    MS_DPP_MAX(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
-#undef MS_DPP_MAX
-    return __builtin_amdgcn_readlane(x, 63);
-}
-
-// Orders a wave's LDS accesses among its lanes (LDS serves one wave in order).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Thread (g, j) holds codes 8 g .. 8 g + 7 of lane j (at most 32 bits each):
 // 8 bw bits that start at byte g bw of the lane's stream.  They are ORed
 // into the block's words (cleared here), two codes at a time and with one
@@ -952,7 +927,7 @@ __global__ __launch_bounds__(OP_WAVES * 64, 4) void k_emit_onepass(emit_layout l
                 uint64_t o = 1;
 #pragma unroll
                 for (uint32_t q = 0; q < 8; q++) o |= x[k][q];
-                bw[k] = wave_max_u32(64 - __clzll(o));
+                bw[k] = dpp_max_u32(64 - __clzll(o));
                 if (KIND == MS_DYNAMIC_VBP) hdr[k] = k == 0 && page0 ? P : 0;
                 else hdr[k] = ((k & (bpo - 1)) == 0 ? P : 0) + (KIND == MS_FOR && k == 0 && page0 ? 8 * FP : 0);
                 bytes += hdr[k] + OP_B / 8 * bw[k];
@@ -1358,11 +1333,6 @@ constexpr uint32_t RLE_WAVES = 8, RLE_ROWS = 16;
 constexpr uint32_t RLE_WV = RLE_ROWS * 128;             // values per wave
 constexpr uint32_t RLE_TILE = RLE_WAVES * RLE_WV;       // values per tile
 constexpr uint32_t RLE_SLOT = 256;                      // heads per wave kept in LDS
-
-__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-}
 
 // The n values at src, two consecutive ones per lane and row; `before` =
 // the value in front of them.
