@@ -55,7 +55,7 @@ struct ms_plan {
     hipGraph_t graph;
     hipGraphExec_t exec;
     bool recording;
-    std::vector<void *> deferred;   // frees of eager memory requested while capturing
+    std::vector<std::pair<void *, bool>> deferred;   // frees of eager memory requested while capturing; may it be kept
     std::vector<std::pair<void (*)(void *), void *>> holds;   // objects the graph reads
 };
 
@@ -807,7 +807,7 @@ extern "C" int ms_col_free(ms_col *c)
     if (c->arena) {
         // arena columns die with their plan
     } else if (plan_capturing()) {
-        g_rec->deferred.push_back((void *)c->meta);   // a free now would be captured into the graph
+        g_rec->deferred.emplace_back((void *)c->meta, !c->unordered);   // a free now would be captured into the graph
     } else {
         free_ordered((void *)c->meta, c->stream, !c->unordered);
     }
@@ -1011,7 +1011,7 @@ extern "C" int ms_plan_end(ms_plan *p, void *stream)
         return MS_OK;
     }
     hipError_t e = hipStreamEndCapture(p->stream, &p->graph);
-    for (void *q : p->deferred) free_ordered(q, p->stream);
+    for (const auto &q : p->deferred) free_ordered(q.first, p->stream, q.second);
     p->deferred.clear();
     if (no_columns()) cache().drop();
     if (e != hipSuccess) return ms_fail(MS_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));

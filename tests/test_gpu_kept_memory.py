@@ -275,3 +275,26 @@ def test_columns_read_by_a_plan():
     del col
     assert used_by_pool() < before + (8 << 20)
     assert len(keep.values()) == 40
+
+
+def test_freed_while_a_plan_captures_after_a_non_blocking_read():
+    nb, res = NonBlocking(), ea.DeviceU64()
+    st, plan = hip.Stream(), ea.Plan()
+    keep = ea.upload_values(np.arange(40, dtype=np.uint64))
+    with plan.record(st):
+        ea.agg_sum(keep, st)
+    ea.release_memory()
+    before = used_by_pool()
+    col = ea.upload_values(np.arange(1 << 20, dtype=np.uint64))
+    hip.synchronize()
+    ea.select_sum(MS_CMP_LT, 9, col, res, nb)
+    nb.synchronize()
+    with plan.record(st):
+        total = ea.agg_sum(keep, st)
+        del col
+    assert used_by_pool() < before + (8 << 20)
+    plan.launch(st)
+    assert int(total.values(st)[0]) == 780 and int(res.get()[0]) == 36
+    del total
+    plan.free()
+    nb.destroy()
